@@ -110,7 +110,8 @@ int jh_ctx_set_flux(jh_ctx* ctx, int solver_type, int split_method, int reconstr
  * tile autotuner (janc_amd/autotune.py).  The Godunov kernel has one tile
  * shape per reconstruction (WENO5_JS: 64 x 3 cells, 256 threads; MUSCL:
  * 64 x 7 cells, 512 threads), the Steger-Warming kernel one (64 x 16 cells,
- * 512 threads). */
+ * 512 threads).  Grids of up to 200000 cells run a kernel of smaller tiles
+ * under LF splitting with WENO5_JS, whatever the variant. */
 int jh_ctx_set_tile(jh_ctx* ctx, int variant);
 int jh_ctx_get_tile(const jh_ctx* ctx);
 

@@ -14,6 +14,7 @@
 #include "adjoint.hpp"
 #include "batch.hpp"
 #include "blocks.hpp"
+#include "compact.hpp"
 #include "godunov.hpp"
 #include "stage.hpp"
 
@@ -36,6 +37,7 @@ struct jh_ctx {
   int parity = 0;
   bool user_filled[4] = {false, false, false, false};   // JH_BC_USER strips written
   int tile = 0;                   // stage-kernel variant (kTileRows / kTileWaves)
+  CompactTile compact{0, 0, 0, 0};   // small grids: the compact kernel's tile (R = 0: none)
   int solver = JH_SOLVER_FLUX_SPLITTING;   // jh_ctx_set_flux
   int split = JH_SPLIT_LF;
   int recon = JH_RECON_WENO5_JS;
@@ -227,6 +229,54 @@ constexpr int kTileWaves[kTileVariants] = {3, 4, 4, 5, 4};
 // rows at a 4-wave register budget, whatever the context's variant.
 constexpr int kGridRows = 16;
 
+// Small grids: the compact stage kernel (compact.hpp) by cell count, whatever
+// the tile variant (which shapes the wide kernel).  Up to 256 tiles of a wave
+// per variable all 12 variables run at once (14336 cells = one block per CU);
+// then two groups of rounds while the chip still holds every block at once
+// (50000 cells); then 2 groups of 256 threads, until the wide kernel has tiles
+// enough for the chip.  Microseconds per FP64 step (wide / compact, G = 12, 6,
+// 2): 4096 cells 155 / 46, 53, 66; 16384: 157 / 60, 58, 70; 25641: 160 / 62,
+// 61, 72; 65536: 166 / 109, 126, 97; 105000: 175 / 158, 165, 103; 262144: 191 /
+// 315, 349, 205.  Mixed: 4096: 121 / 45, 51, 65; 25641: 126 / 60, 59, 71; 65536:
+// 131 / 104, 118, 87; 105000: 139 / 142, 151, 93; 262144: 157 / 293, 322, 164.
+struct CompactRule { int groups, threads, halo; long long cells; };
+constexpr CompactRule kCompactRules[3] = {{12, 64, 2, 14336}, {6, 128, 2, 50000},
+                                          {2, 256, 1, 200000}};
+
+int compact_rule(const jh_ctx* c) {
+  const long long n = (long long)c->nx * c->ny;
+  for (int k = 0; k < 3; ++k)
+    if (n <= kCompactRules[k].cells) return k;
+  return -1;
+}
+
+template <typename Real, int K>
+void launch_compact_rule(jh_ctx* c, const StepArgs<Real>& a, int stage, const Real* Us,
+                         const Real* As, const Real* Un, Real* Uo, Real* Ao) {
+  constexpr CompactRule r = kCompactRules[K];
+  constexpr int NT = r.groups * r.threads;
+  const CompactTile& ct = c->compact;
+  const int nb = ct.tiles_x * ct.tiles_y;
+  const size_t lds = compact_lds<r.groups>(ct) * sizeof(Real);
+  if (a.mirror)
+    compact_stage_kernel<Real, MODE_RK, r.groups, r.halo, NT, ADDR_MIRROR>
+        <<<nb, NT, lds, c->stream>>>(a, ct, r.threads, stage, Us, As, Un, Uo, Ao);
+  else
+    compact_stage_kernel<Real, MODE_RK, r.groups, r.halo, NT, ADDR_STRIP>
+        <<<nb, NT, lds, c->stream>>>(a, ct, r.threads, stage, Us, As, Un, Uo, Ao);
+}
+
+template <typename Real>
+void launch_compact(jh_ctx* c, const StepArgs<Real>& a, int stage, const Real* Us, const Real* As,
+                    const Real* Un, Real* Uo, Real* Ao) {
+  switch (compact_rule(c)) {
+    case 0: launch_compact_rule<Real, 0>(c, a, stage, Us, As, Un, Uo, Ao); break;
+    case 1: launch_compact_rule<Real, 1>(c, a, stage, Us, As, Un, Uo, Ao); break;
+    case 2: launch_compact_rule<Real, 2>(c, a, stage, Us, As, Un, Uo, Ao); break;
+    default: break;
+  }
+}
+
 template <typename Real, int MODE, int RECON>
 void launch_split_stage(jh_ctx* c, const StepArgs<Real>& a, int stage, const Real* Us,
                         const Real* As, const Real* Un, Real* Uo, Real* Ao) {
@@ -235,6 +285,12 @@ void launch_split_stage(jh_ctx* c, const StepArgs<Real>& a, int stage, const Rea
     stage_kernel<Real, MODE, kGridRows, 4, RECON, SPLIT_LF, Real, true>
         <<<nbg, Tile<kGridRows>::NT, 0, c->stream>>>(a, stage, Us, As, Un, Uo, Ao);
     return;
+  }
+  if constexpr (MODE == MODE_RK && RECON == RECON_WENO5) {
+    if (c->compact.R > 0) {
+      launch_compact<Real>(c, a, stage, Us, As, Un, Uo, Ao);
+      return;
+    }
   }
   const int nb = stage_blocks(c);
   switch (c->tile) {
@@ -1121,6 +1177,9 @@ int jh_ctx_create(int nx, int ny, double dx, double dy, const int* bc_kind,
   // 16 rows with the 5-wave register budget for FP64, 16 rows at 4 waves/SIMD
   // for the mixed form
   c->tile = precision == JH_PREC_FP64 ? 3 : 2;
+  const int rule = compact_rule(c);
+  if (rule >= 0)
+    c->compact = compact_tile(nx, ny, kCompactRules[rule].threads, kCompactRules[rule].halo);
   c->stream = static_cast<hipStream_t>(stream);
   for (int s = 0; s < 4; ++s) {
     c->bc[s] = bc_kind[s];
