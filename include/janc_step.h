@@ -398,6 +398,20 @@ int jh_blocks_stage_noalloc(jh_blocks* blocks, int n_blk, int stage, const void*
  * interior blocks (n_blk, 14, bnx, bny): U += reaction_source_terms(U, aux,
  * dt) (reaction_model.py:183-203), aux = update_aux(U, aux). */
 int jh_blocks_chem(jh_blocks* blocks, int n_blk, void* blk, double dt);
+/* One whole step of a uniform level (advance_one_step_amr, TVD_RK3.py:15-37,
+ * and the chemistry branch, set_simulator.py:107-111) without padded copies:
+ * the interior blocks blk (n_blk blocks read through the element strides sb
+ * (block), sv (plane) and sr (row), columns contiguous) -> out (n_blk, 14, bnx,
+ * bny), contiguous, not aliasing blk.  idx, s_u, s_v: the level's ghost tables
+ * as jh_blocks_fill_ghosts takes them.  work: jh_blocks_level_work(n_blk) bytes
+ * of device memory, 256-byte aligned, used during the call's kernels only.
+ * Equals jh_blocks_fill_ghosts + jh_blocks_stage three times and
+ * jh_blocks_chem bit for bit on the interiors; the health flags are the
+ * interior cells' (the ghost copies are not updated). */
+long long jh_blocks_level_work(const jh_blocks* blocks, int n_blk);
+int jh_blocks_level_step(jh_blocks* blocks, int n_blk, const void* blk, long long sb,
+                         long long sv, long long sr, const int* idx, const void* s_u,
+                         const void* s_v, double dt, void* work, void* out);
 /* OR of every block's health flags since the last call; synchronises. */
 int jh_blocks_health(jh_blocks* blocks, unsigned int* flags);
 

@@ -99,6 +99,9 @@ SIGNATURES = {
     "jh_blocks_stage": (_c_int, [_vp, _c_int, _c_int, _vp, _vp, _c_double, _vp]),
     "jh_blocks_stage_noalloc": (_c_int, [_vp, _c_int, _c_int, _vp, _vp, _c_double, _vp]),
     "jh_blocks_chem": (_c_int, [_vp, _c_int, _vp, _c_double]),
+    "jh_blocks_level_work": (ctypes.c_longlong, [_vp, _c_int]),
+    "jh_blocks_level_step": (_c_int, [_vp, _c_int, _vp, ctypes.c_longlong, ctypes.c_longlong,
+                                      ctypes.c_longlong, _vp, _vp, _vp, _c_double, _vp, _vp]),
     "jh_blocks_health": (_c_int, [_vp, ctypes.POINTER(ctypes.c_uint)]),
 }
 

@@ -135,6 +135,8 @@ class BlockSolver:
         if amr is None:
             raise ValueError("advance_one_step needs the AMR hierarchy's ghost functions "
                              "(jaxamr's amr module or an object with the same two functions)")
+        if type(amr) is UniformBlockGrid and ref_blk_data.is_cuda:
+            return self._level_step(amr, ref_blk_data, dx, dy, dt)
         g0 = amr.get_ghost_block_data(ref_blk_data, ref_blk_info)
         b = None
         gs = g0
@@ -145,6 +147,23 @@ class BlockSolver:
                 gs = amr.get_ghost_block_data(b, ref_blk_info)
         b = b.contiguous()
         return self.chemistry(b, dx, dy, dt)
+
+    def _level_step(self, grid, blk, dx, dy, dt):
+        """advance_one_step on a uniform level's own grid: the library's level
+        kernels read the interiors through the grid's tables
+        (jh_blocks_level_step) instead of refilled padded copies."""
+        su, sv = grid.gpu_tables(blk)
+        if blk.dtype != self.dtype:
+            raise TypeError("blocks must be contiguous %s CUDA tensors" % self.dtype)
+        ctx = self._blocks(grid.bnx, grid.bny, dx, dy)
+        n = int(blk.shape[0])
+        work = torch.empty((ctx.lib.jh_blocks_level_work(ctx.h, n),), dtype=torch.uint8,
+                           device=blk.device)
+        out = torch.empty(tuple(blk.shape), dtype=blk.dtype, device=blk.device)
+        ctx.call("jh_blocks_level_step", n, _ptr(blk), blk.stride(0), blk.stride(1),
+                 blk.stride(2), _ptr(grid._idx32), _ptr(su), _ptr(sv), float(dt), _ptr(work),
+                 _ptr(out))
+        return out
 
     def health(self):
         """OR of every block context's health flags since the last query."""
@@ -275,8 +294,9 @@ class UniformBlockGrid:
         full = b.permute(2, 0, 3, 1, 4).reshape(nv, self.nbx * self.bnx, self.nby * self.bny)
         return full[:-2], full[-2:]
 
-    def _fill_gpu(self, blk):
-        from .solver import _ptr
+    def gpu_tables(self, blk):
+        """Momentum signs in blk's type, after checking that blk is this
+        level's interiors on the grid's device."""
         if blk.dtype not in (torch.float64, torch.float32) or blk.dim() != 4 \
                 or tuple(blk.shape) != (self.n_blk, 14, self.bnx, self.bny) \
                 or blk.stride(3) != 1 or blk.device != self._idx32.device:
@@ -286,7 +306,10 @@ class UniformBlockGrid:
         if blk.dtype not in self._signs:
             self._signs[blk.dtype] = (self.s_u.to(blk.dtype).contiguous(),
                                       self.s_v.to(blk.dtype).contiguous())
-        su, sv = self._signs[blk.dtype]
+        return self._signs[blk.dtype]
+
+    def _fill_gpu(self, blk):
+        su, sv = self.gpu_tables(blk)
         out = torch.empty((self.n_blk, 14, self.bnx + 6, self.bny + 6), dtype=blk.dtype,
                           device=blk.device)
         lib = _lib.load()

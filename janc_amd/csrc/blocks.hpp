@@ -13,13 +13,20 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "compact.hpp"
 #include "stage.hpp"
 
 namespace jh {
 
-// Rows of the block stage kernel's tile: AMR blocks are small (tens of cells
-// per side), so the short tile wastes the fewest rows.
-constexpr int kBlkRows = 8;
+// Threads of a block stage kernel at most: tiles of up to 256 faces, sized to
+// the AMR block (compact_tile).  Several small workgroups per CU cover one
+// another's barriers: a whole FP64 step of 2500 blocks of 20 x 20 (a level in
+// place) takes 694 us at 256 or 384 threads, 745 at 512, 799 at 192; the mixed
+// step of 1000 blocks of 40 x 50 943 us at 256, 954 at 192, 1145 at 512.
+constexpr int kBlkThreads = 256;
+// Waves per SIMD its register budget allows (FP32 needs 80 registers).
+template <typename Real> struct BlkWaves { static constexpr int value = 4; };
+template <> struct BlkWaves<float> { static constexpr int value = 6; };
 
 // LF maxima of stage `stage` of every block over its padded field
 // (LF.py:10-11 under vmap): one workgroup per block, stored (not folded) into
@@ -59,25 +66,93 @@ __global__ __launch_bounds__(256) void blocks_alpha_kernel(StepArgs<Real> a, int
 }
 
 // One RK stage (MODE_RK) or the flux_func alone (MODE_RHS) of every block's
-// interior: the stage kernel body on a block's padded planes, the block's
+// interior: the compact stage body on a block's padded planes, the block's
 // own maxima.  Jobs (block, tile) in XCD-contiguous order.  bs / bo: block
 // strides of the inputs and of the output (12 planes per block for MODE_RHS).
-template <typename Real, int MODE, int TX, int WPE>
-__global__ __launch_bounds__(Tile<TX>::NT) __attribute__((amdgpu_waves_per_eu(WPE)))
-void blocks_stage_kernel(StepArgs<Real> a, int stage, int tiles_per_blk, long long bs,
-                         long long bo, const Real* Bs, const Real* Bn, Real* Bo) {
-  __shared__ StageLds<Real, TX> L;
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
-  const int b = t / tiles_per_blk, tile = t - b * tiles_per_blk;
+// Bound by FP64 issue; the 64-column tile it replaced left 44 of 64 lanes of a
+// 20 x 20 block idle.
+template <typename Real, int MODE>
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(BlkWaves<Real>::value)))
+void blocks_stage_kernel(StepArgs<Real> a, CompactTile ct, int stage, long long bs, long long bo,
+                         const Real* Bs, const Real* Bn, Real* Bo) {
+  extern __shared__ double dyn[];
+  __shared__ MixTables mix;
+  __shared__ double red[32];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), tiles = ct.tiles_x * ct.tiles_y;
+  const int b = t / tiles, tile = t - b * tiles;
   const size_t P = (size_t)(a.nx + 6) * (a.ny + 6);
   StepArgs<Real> ab = a;
   ab.sc = a.sc + b;
   ab.parity = 0;
   const Real* Us = Bs + (size_t)b * bs;
-  const Real* Un = Bn + (size_t)b * bs;
   Real* Uo = Bo + (size_t)b * bo;
-  stage_body<Real, MODE, TX, RECON_WENO5, SPLIT_LF, Real, false, true>(
-      ab, stage, Us, Us + NU * P, Un, Uo, Uo + NU * P, tile, L);
+  compact_body<Real, MODE, 1, 1, ADDR_PAD>(ab, ct, stage, Us, Us + NU * P, Bn + (size_t)b * bs, Uo,
+                                           Uo + NU * P, tile, blockDim.x,
+                                           reinterpret_cast<Real*>(dyn), mix, red);
+}
+
+// One RK stage of a uniform level's blocks read in place: the halo of a block
+// comes from the other blocks' interiors through the level's index table and
+// the output is the interiors alone, so no padded copy is filled and no ghost
+// ring is written (lv: tables and strides; Uo: (n_blk, 14, nx, ny)).
+template <typename Real>
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(BlkWaves<Real>::value)))
+void level_stage_kernel(StepArgs<Real> a, CompactTile ct, int stage, LevelMap<Real> lv,
+                        const Real* Us, const Real* Un, Real* Uo) {
+  extern __shared__ double dyn[];
+  __shared__ MixTables mix;
+  __shared__ double red[32];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), tiles = ct.tiles_x * ct.tiles_y;
+  const int b = t / tiles, tile = t - b * tiles;
+  const size_t n = (size_t)a.nx * a.ny;
+  StepArgs<Real> ab = a;
+  ab.sc = a.sc + b;
+  Real* Ub = Uo + (size_t)b * (NU + 2) * n;
+  compact_body<Real, MODE_RK, 1, 1, ADDR_LEVEL>(ab, ct, stage, Us, nullptr, Un, Ub, Ub + NU * n,
+                                                tile, blockDim.x, reinterpret_cast<Real*>(dyn),
+                                                mix, red, &lv, b);
+}
+
+// |u| + a and |v| + a of every interior cell of a level (two planes of ncell)
+// and each block's maxima of them into its stage-0 slots (the later stages'
+// slots are cleared): what the level's stage kernels take the LF maxima from.
+// One workgroup per block.
+template <typename Real>
+__global__ __launch_bounds__(256) void level_speeds_kernel(StepArgs<Real> a, long long sb,
+                                                           long long splane, long long sr,
+                                                           const Real* __restrict__ U,
+                                                           double* __restrict__ spd, int ncell) {
+  __shared__ double red[8];
+  const int n = a.nx * a.ny, b = blockIdx.x;
+  double mx = 0.0, my = 0.0;
+  for (int l = threadIdx.x; l < n; l += blockDim.x) {
+    const int x = l / a.ny, i = b * n + l;
+    const Real* p = U + b * sb + x * sr + (l - x * a.ny);
+    const Prim<double> q = cell_prim<double, true>(*a.mc, p, p + NU * splane, (int)splane);
+    const double sx = nan_to_zero(fabs(q.u) + q.a), sy = nan_to_zero(fabs(q.v) + q.a);
+    spd[i] = sx;
+    spd[ncell + i] = sy;
+    mx = fmax(mx, sx);
+    my = fmax(my, sy);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    mx = fmax(mx, __shfl_xor(mx, off, 64));
+    my = fmax(my, __shfl_xor(my, off, 64));
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0) {
+    red[wid] = mx;
+    red[4 + wid] = my;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double m = red[4 * threadIdx.x];
+    for (int w = 1; w < 4; ++w) m = fmax(m, red[4 * threadIdx.x + w]);
+    a.sc[b].amax[0][0][threadIdx.x] = dbits(m);
+    a.sc[b].amax[0][1][threadIdx.x] = 0ull;
+    a.sc[b].amax[0][2][threadIdx.x] = 0ull;
+  }
 }
 
 // The ghost layers of a stage's output blocks, as the reference computes
@@ -153,23 +228,17 @@ __global__ __launch_bounds__(256) void blocks_ring_kernel(StepArgs<Real> a, int 
 }
 
 // Chemistry and final update_aux of every block's interior, in place
-// (set_simulator.py:107-111): blocks (n_blk, 14, nx, ny).  Grid: (cells /
-// 256, n_blk).
+// (set_simulator.py:107-111): blocks (n_blk, 14, nx, ny).  Grid: all cells /
+// 256 (a grid of whole workgroups per block left a fifth of the lanes idle at
+// 400 cells a block).
 template <typename Real>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void blocks_chem_kernel(StepArgs<Real> a, long long bs, Real* B) {
-  __shared__ double red[4];
-  __shared__ unsigned long long redb[4];
-  __shared__ unsigned long long redg[kGridSlotsChem * 4];
+void blocks_chem_kernel(StepArgs<Real> a, long long bs, Real* B, int n_blk) {
   __shared__ MixTables mix;
   __shared__ GibbsTables gt;
-  const int b = blockIdx.y;
-  StepArgs<Real> ab = a;
-  ab.sc = a.sc + b;
-  ab.parity = 0;
-  Real* U = B + (size_t)b * bs;
-  chem_body<Real, CHEM_STEP>(ab, U, U + (size_t)NU * a.nx * a.ny, nullptr, nullptr, blockIdx.x,
-                             red, redb, redg, mix, gt);
+  chem_body<Real, CHEM_STEP, false, false, true>(a, B, B + (size_t)NU * a.nx * a.ny, nullptr,
+                                                 nullptr, blockIdx.x, nullptr, nullptr, nullptr,
+                                                 mix, gt, bs, n_blk);
 }
 
 // Ghost refill of same-size blocks tiling one uniform level: out[b][v][p]

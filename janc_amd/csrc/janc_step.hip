@@ -1103,6 +1103,12 @@ StepArgs<Real> blocks_args(const jh_blocks* b, double dt, StepScalars* sc) {
   return a;
 }
 
+// Threads of a block stage kernel: one per x face, y face, cell and halo cell.
+int blk_threads(const CompactTile& ct) {
+  const int m = std::max(std::max(ct.fx(), ct.fy()), ct.halo());
+  return (m + 63) / 64 * 64;
+}
+
 template <typename Real, int MODE>
 int blocks_stage_impl(jh_blocks* b, int n_blk, int stage, const Real* Bs, const Real* Bn,
                       Real* Bo, double dt, StepScalars* sc) {
@@ -1111,14 +1117,67 @@ int blocks_stage_impl(jh_blocks* b, int n_blk, int stage, const Real* Bs, const 
   auto a = blocks_args<Real>(b, dt, sc);
   hipStream_t st = b->stream;
   blocks_alpha_kernel<Real><<<n_blk, 256, 0, st>>>(a, stage, bs, Bs);
-  const int tiles = ((b->nx + kBlkRows - 1) / kBlkRows) * ((b->ny + TY - 1) / TY);
-  blocks_stage_kernel<Real, MODE, kBlkRows, 4>
-      <<<n_blk * tiles, Tile<kBlkRows>::NT, 0, st>>>(a, stage, tiles, bs, bo, Bs, Bn, Bo);
+  const CompactTile ct = compact_tile(b->nx, b->ny, kBlkThreads, 1);
+  blocks_stage_kernel<Real, MODE>
+      <<<n_blk * ct.tiles_x * ct.tiles_y, blk_threads(ct), compact_lds<1>(ct) * sizeof(Real), st>>>(
+          a, ct, stage, bs, bo, Bs, Bn, Bo);
   const int nring = (int)(P - (long long)b->nx * b->ny);
   blocks_ring_kernel<Real, MODE>
       <<<dim3((nring + 255) / 256, n_blk), 256, 0, st>>>(a, stage, bs, bo, Bs, Bn, Bo);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kfail(b, JH_ERR_HIP, std::string("block kernels: ") +
+                                                       hipGetErrorString(e));
+  return JH_OK;
+}
+
+template <typename Real>
+void launch_blocks_chem(jh_blocks* b, int n_blk, Real* blk, double dt) {
+  const int n = b->nx * b->ny;
+  const int nb = (int)(((long long)n * n_blk + 255) / 256);
+  blocks_chem_kernel<Real><<<nb, 256, 0, b->stream>>>(blocks_args<Real>(b, dt, b->sc),
+                                                      (long long)(NU + 2) * n, blk, n_blk);
+}
+
+// Bytes of one state and of the speeds of a level's work area.
+size_t level_state(const jh_blocks* b, int n_blk) {
+  const size_t es = b->precision == JH_PREC_FP64 ? 8 : 4;
+  return (((size_t)n_blk * (NU + 2) * b->nx * b->ny * es) + 255) / 256 * 256;
+}
+size_t level_speeds(const jh_blocks* b, int n_blk) {
+  return ((size_t)n_blk * b->nx * b->ny * 2 * sizeof(double) + 255) / 256 * 256;
+}
+
+template <typename Real>
+int level_step_impl(jh_blocks* b, int n_blk, const Real* blk, long long sb, long long sv,
+                    long long sr, const int* idx, const Real* su, const Real* svg, double dt,
+                    char* work, Real* out) {
+  const int n = b->nx * b->ny, ncell = n_blk * n;
+  const size_t ss = level_state(b, n_blk), sp = level_speeds(b, n_blk);
+  Real* mid[2] = {reinterpret_cast<Real*>(work), reinterpret_cast<Real*>(work + ss)};
+  double* spd[2] = {reinterpret_cast<double*>(work + 2 * ss),
+                    reinterpret_cast<double*>(work + 2 * ss + sp)};
+  hipStream_t st = b->stream;
+  const auto a = blocks_args<Real>(b, dt, b->sc);
+  const CompactTile ct = compact_tile(b->nx, b->ny, kBlkThreads, 1);
+  const int nb = n_blk * ct.tiles_x * ct.tiles_y, nt = blk_threads(ct);
+  const size_t lds = compact_lds<1>(ct) * sizeof(Real);
+  level_speeds_kernel<Real><<<n_blk, 256, 0, st>>>(a, sb, sv, sr, blk, spd[0], ncell);
+  const long long ob = (long long)(NU + 2) * n;
+  LevelMap<Real> lv{idx, su, svg, spd[0], spd[1], sb, sv, sr, sb, sv, sr, ncell};
+  const Real* src = blk;
+  Real* dst[3] = {mid[0], mid[1], out};
+  for (int s = 0; s < 3; ++s) {
+    lv.spd = spd[s & 1];
+    lv.spd_out = s < 2 ? spd[(s + 1) & 1] : nullptr;
+    level_stage_kernel<Real><<<nb, nt, lds, st>>>(a, ct, s, lv, src, blk, dst[s]);
+    src = dst[s];
+    lv.sb = ob;
+    lv.splane = n;
+    lv.sr = b->ny;
+  }
+  launch_blocks_chem<Real>(b, n_blk, out, dt);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return kfail(b, JH_ERR_HIP, std::string("level kernels: ") +
                                                        hipGetErrorString(e));
   return JH_OK;
 }
@@ -1979,19 +2038,36 @@ int jh_blocks_chem(jh_blocks* b, int n_blk, void* blk, double dt) {
   if (!(dt > 0)) return kfail(b, JH_ERR_ARG, "dt must be > 0");
   int rc = blocks_checks(b, n_blk);
   if (rc) return rc;
-  const int n = b->nx * b->ny;
-  const long long bs = (long long)(NU + 2) * n;
-  const dim3 grid((n + 255) / 256, n_blk);
-  if (b->precision == JH_PREC_FP64)
-    blocks_chem_kernel<double><<<grid, 256, 0, b->stream>>>(blocks_args<double>(b, dt, b->sc),
-                                                            bs, (double*)blk);
-  else
-    blocks_chem_kernel<float><<<grid, 256, 0, b->stream>>>(blocks_args<float>(b, dt, b->sc), bs,
-                                                           (float*)blk);
+  if (b->precision == JH_PREC_FP64) launch_blocks_chem<double>(b, n_blk, (double*)blk, dt);
+  else launch_blocks_chem<float>(b, n_blk, (float*)blk, dt);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kfail(b, JH_ERR_HIP, std::string("block chemistry: ") +
                                                        hipGetErrorString(e));
   return JH_OK;
+}
+
+long long jh_blocks_level_work(const jh_blocks* b, int n_blk) {
+  if (!b || n_blk < 1) return 0;
+  return (long long)(2 * level_state(b, n_blk) + 2 * level_speeds(b, n_blk));
+}
+
+int jh_blocks_level_step(jh_blocks* b, int n_blk, const void* blk, long long sb, long long sv,
+                         long long sr, const int* idx, const void* s_u, const void* s_v,
+                         double dt, void* work, void* out) {
+  if (!b) return JH_ERR_ARG;
+  if (!blk || !idx || !s_u || !s_v || !work || !out) return kfail(b, JH_ERR_ARG, "NULL pointer");
+  if (out == blk) return kfail(b, JH_ERR_ARG, "out must not alias the blocks");
+  if (!(dt > 0)) return kfail(b, JH_ERR_ARG, "dt must be > 0");
+  if (sb < 1 || sv < 1 || sr < b->ny || sv >= (1ll << 31))
+    return kfail(b, JH_ERR_ARG, "bad strides");
+  int rc = blocks_checks(b, n_blk);
+  if (rc) return rc;
+  if (b->precision == JH_PREC_FP64)
+    return level_step_impl<double>(b, n_blk, (const double*)blk, sb, sv, sr, idx,
+                                   (const double*)s_u, (const double*)s_v, dt, (char*)work,
+                                   (double*)out);
+  return level_step_impl<float>(b, n_blk, (const float*)blk, sb, sv, sr, idx, (const float*)s_u,
+                                (const float*)s_v, dt, (char*)work, (float*)out);
 }
 
 int jh_blocks_health(jh_blocks* b, unsigned int* flags) {

@@ -1302,12 +1302,15 @@ struct MemState {
 // plus the next step's CFL and stage-1 LF maxima.  CHEM_SOURCE writes the
 // source S (12 planes, first 4 zero) instead.  GRID: the grid-wide Halley
 // stop's epilogue (a.hside set), compiled apart so that the per-cell form
-// keeps its registers.
-template <typename Real, int MODE, bool REPLAY = false, bool GRID = false>
+// keeps its registers.  BLOCKS: U and aux are the first of nblk AMR blocks, bs
+// elements apart, whose cells are dealt to the threads without a gap between
+// blocks (a.sc: one StepScalars per block, flags only; no maxima).
+template <typename Real, int MODE, bool REPLAY = false, bool GRID = false, bool BLOCKS = false>
 __device__ __forceinline__ void chem_body(const StepArgs<Real>& a, Real* U, Real* aux, Real* S,
                                           double* dt_hist, int blk, double* red,
                                           unsigned long long* redb, unsigned long long* redg,
-                                          MixTables& mix, GibbsTables& gt) {
+                                          MixTables& mix, GibbsTables& gt, long long bs = 0,
+                                          int nblk = 1) {
   const MechConst& c = *a.mc;
   if (MODE == CHEM_STEP) load_mix_tables(c, mix);
   load_gibbs_tables(c, gt);
@@ -1323,8 +1326,13 @@ __device__ __forceinline__ void chem_body(const StepArgs<Real>& a, Real* U, Real
   unsigned int fl = 0u;
   // one cell per thread: a grid-stride loop would let the compiler keep every
   // mechanism constant in registers across iterations
-  const int i = blk * blockDim.x + threadIdx.x;
-  if (i < n) {
+  const int it = blk * blockDim.x + threadIdx.x;
+  const int b = BLOCKS ? it / n : 0, i = it - b * n;
+  if (BLOCKS) {
+    U += b * bs;
+    aux += b * bs;
+  }
+  if (BLOCKS ? b < nblk : i < n) {
     // the state is read before the Jacobian and again after the solve
     // instead of being held across it
     const MemState<Real> ld{U, n, i};
@@ -1398,7 +1406,9 @@ __device__ __forceinline__ void chem_body(const StepArgs<Real>& a, Real* U, Real
       cm = b > cm ? b : cm;
     }
   }
-  if (MODE == CHEM_STEP) {
+  if constexpr (BLOCKS) {
+    if (fl) atomicOr(&a.sc[b].flags, fl);
+  } else if (MODE == CHEM_STEP) {
     raise_flags(a.sc, fl);
     const int o = a.parity ^ 1;
     if constexpr (grid) {
