@@ -89,7 +89,9 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
   }
   const int x0 = (tile / ct.tiles_y) * R, y0 = (tile % ct.tiles_y) * C;
   const double dt = step_dt(a);
-  const double idx = 1.0 / a.dx, idy = 1.0 / a.dy;
+  constexpr double sc = LfScale<W>::value;   // split fluxes scaled as stage_body's
+  constexpr W hs = (W)(0.5 * sc);
+  const double idx = 1.0 / sc / a.dx, idy = 1.0 / sc / a.dy;
   double alx, aly;
   if constexpr (ADDR == ADDR_LEVEL) {
     // the block's LF maxima: its interior cells' (reduced by the producer) and
@@ -130,7 +132,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
     alx = bitsd(a.sc->amax[a.parity][stage][0]);
     aly = bitsd(a.sc->amax[a.parity][stage][1]);
   }
-  const W hax = (W)0.5 * (W)(Real)alx, hay = (W)0.5 * (W)(Real)aly;
+  const W hax = hs * (W)(Real)alx, hay = hs * (W)(Real)aly;
 
   // ---- the thread's cells: slot 0 = interior cell tg, then halo cells ----
   constexpr int NS = 1 + NH;
@@ -277,7 +279,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
       if (s == 0 || xhalo[s]) {
         W hp = (W)0, hm = (W)0;
         if (ref[s].ok) {
-          const W hF = (W)0.5 * phys_flux<W>(CLS, 0, q[s], ucv);
+          const W hF = hs * phys_flux<W>(CLS, 0, q[s], ucv);
           hp = fma(hax, ucv, hF);
           hm = fma(-hax, ucv, hF);
         }
@@ -287,7 +289,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
       if (s == 0 || !xhalo[s]) {
         W hp = (W)0, hm = (W)0;
         if (ref[s].ok) {
-          const W hG = (W)0.5 * phys_flux<W>(CLS, 1, q[s], ucv);
+          const W hG = hs * phys_flux<W>(CLS, 1, q[s], ucv);
           hp = fma(hay, ucv, hG);
           hm = fma(-hay, ucv, hG);
         }
@@ -328,13 +330,13 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
     if (xface) {
       const W* p = sHxp + tg;
       const W* m = sHxm + tg;
-      sFx[tg] = weno5(p[0], p[C], p[2 * C], p[3 * C], p[4 * C]) +
-                weno5(m[5 * C], m[4 * C], m[3 * C], m[2 * C], m[C]);
+      sFx[tg] = weno5_lf(p[0], p[C], p[2 * C], p[3 * C], p[4 * C], m[C], m[2 * C], m[3 * C],
+                         m[4 * C], m[5 * C]);
     }
     if (yface) {
       const W* p = sHyp + ybase;
       const W* m = sHym + ybase;
-      sFy[tg] = weno5(p[0], p[1], p[2], p[3], p[4]) + weno5(m[5], m[4], m[3], m[2], m[1]);
+      sFy[tg] = weno5_lf(p[0], p[1], p[2], p[3], p[4], m[1], m[2], m[3], m[4], m[5]);
     }
     __syncthreads();
     // ---- phase 3: divergence + RK combine, as stage_body ----

@@ -916,6 +916,17 @@ __device__ __forceinline__ void sw_split(int cv, int dir, const Prim<W>& q, W uc
   hm = (W)0.5 * (l1 - s1) * H1 + (W)0.5 * (l2 - s2) * H2 + (W)0.5 * (l4 - s4) * H4;
 }
 
+// Flux at one face: left-biased value of H+ plus right-biased value of H-,
+// whose stencils start at p and m (stride s).
+template <int RECON, int SPLIT, typename W>
+__device__ __forceinline__ W face_sum(const W* p, const W* m, int s) {
+  if constexpr (RECON == RECON_WENO5 && SPLIT == SPLIT_LF)
+    return weno5_lf(p[0], p[s], p[2 * s], p[3 * s], p[4 * s], m[s], m[2 * s], m[3 * s], m[4 * s],
+                    m[5 * s]);
+  return recon_L<RECON, W>(p[0], p[s], p[2 * s], p[3 * s], p[4 * s]) +
+         recon_R<RECON, W>(m[s], m[2 * s], m[3 * s], m[4 * s], m[5 * s]);
+}
+
 // One SSP-RK3 stage (TVD_RK3.py:5-12) for a 64 x TX tile:
 //   rhs = dt * -(dF/dx + dG/dy)   (set_simulator.py:44-47, flux.py:56-68)
 //   stage 0: U1 = U + rhs; stage 1: U2 = 3/4 U + 1/4 (U1 + rhs);
@@ -990,12 +1001,17 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
   const int x0 = (tile / tiles_y) * TX;
   const int y0 = (tile % tiles_y) * TY;
   const double dt = step_dt(a);
-  const double idx = 1.0 / a.dx, idy = 1.0 / a.dy;
+  // Lax-Friedrichs split fluxes with WENO5 are held scaled (LfScale), undone in
+  // the divergence
+  constexpr double sc =
+      RECON == RECON_WENO5 && SPLIT == SPLIT_LF ? LfScale<W>::value : 1.0;
+  constexpr W hs = (W)(0.5 * sc);
+  const double idx = 1.0 / sc / a.dx, idy = 1.0 / sc / a.dy;
   const W ax = (W)(Real)bitsd(a.sc->amax[a.parity][stage][0]);
   const W ay = (W)(Real)bitsd(a.sc->amax[a.parity][stage][1]);
   // H+- = (F +- alpha U) / 2 as fma(+-alpha/2, U, F/2): halving is exact, so
   // this is the same value with one operation fewer per pair
-  const W hax = (W)0.5 * ax, hay = (W)0.5 * ay;
+  const W hax = hs * ax, hay = hs * ay;
 
   int rrow[NSL], rcol[NSL];       // LDS coordinates: x-region row / y-region col
   int gxs[NSL], gys[NSL];
@@ -1080,7 +1096,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
           if (SPLIT == SPLIT_SW) {
             sw_split<W>(CLS, 0, q[s], ucv, hp, hm);
           } else {
-            const W hF = (W)0.5 * phys_flux<W>(CLS, 0, q[s], ucv);
+            const W hF = hs * phys_flux<W>(CLS, 0, q[s], ucv);
             hp = fma(hax, ucv, hF);
             hm = fma(-hax, ucv, hF);
           }
@@ -1094,7 +1110,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
           if (SPLIT == SPLIT_SW) {
             sw_split<W>(CLS, 1, q[s], ucv, hp, hm);
           } else {
-            const W hG = (W)0.5 * phys_flux<W>(CLS, 1, q[s], ucv);
+            const W hG = hs * phys_flux<W>(CLS, 1, q[s], ucv);
             hp = fma(hay, ucv, hG);
             hm = fma(-hay, ucv, hG);
           }
@@ -1154,21 +1170,13 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
     for (int it = t; it < NXF + NYF; it += NT) {
       if (it < NXF) {
         const int fr = it >> 6, col = it & 63;
-        const W L = recon_L<RECON, W>(sHxp[fr][col], sHxp[fr + 1][col], sHxp[fr + 2][col],
-                                            sHxp[fr + 3][col], sHxp[fr + 4][col]);
-        const W R = recon_R<RECON, W>(sHxm[fr + 1][col], sHxm[fr + 2][col],
-                                            sHxm[fr + 3][col], sHxm[fr + 4][col],
-                                            sHxm[fr + 5][col]);
-        sFx[fr][col] = L + R;
+        const W* p = &sHxp[fr][col];
+        const W* m = &sHxm[fr][col];
+        sFx[fr][col] = face_sum<RECON, SPLIT, W>(p, m, TY);
       } else {
         const int j = it - NXF;
         const int xr = j / (TY + 1), fc = j - xr * (TY + 1);
-        const W L = recon_L<RECON, W>(sHyp[xr][fc], sHyp[xr][fc + 1], sHyp[xr][fc + 2],
-                                            sHyp[xr][fc + 3], sHyp[xr][fc + 4]);
-        const W R = recon_R<RECON, W>(sHym[xr][fc + 1], sHym[xr][fc + 2],
-                                            sHym[xr][fc + 3], sHym[xr][fc + 4],
-                                            sHym[xr][fc + 5]);
-        sFy[xr][fc] = L + R;
+        sFy[xr][fc] = face_sum<RECON, SPLIT, W>(&sHyp[xr][fc], &sHym[xr][fc], 1);
       }
     }
     __syncthreads();

@@ -12,37 +12,70 @@
 
 namespace jh {
 
-// FP64 form.  With the first differences d and the second differences b
-// around f0 (d0 = f0 - fm1, d1 = fp1 - f0, b_k centred on fm1, f0, fp1), the
-// WENO5_JS.py:17-33 smoothness indicators and candidates are
-//   IS_1 = (b_-1/2 + d0)^2 + 13/12 b_-1^2,   q_1 = f0 + b_-1/3 + d0/2
-//   IS_2 = ((d0 + d1)/2)^2 + 13/12 b_0^2,    q_2 = f0 - b_0/6 + d1/2
-//   IS_3 = (b_+1/2 - d1)^2 + 13/12 b_+1^2,   q_3 = f0 - b_+1/6 + d1/2
-// (a_1 = b_-1 + 2 d0, a_2 = -(d0 + d1), a_3 = b_+1 - 2 d1 in the reference's
-// terms).  w_k = alpha_k / sum(alpha) is evaluated as
-// C_k prod_{j!=k} e_j / sum_m C_m prod_{j!=m} e_j with e_k = (eps+IS_k)^2,
-// the same ratio with one reciprocal instead of six divisions, and the value
-// as f0 + sum_k w_k (q_k - f0).  44 FP64 operations per face.
-__host__ __device__ __forceinline__ double weno5(double fm2, double fm1, double f0,
-                                                 double fp1, double fp2) {
-  const double dA = fm1 - fm2, dB = f0 - fm1, dC = fp1 - f0, dD = fp2 - fp1;
-  const double bA = dB - dA, bB = dC - dB, bC = dD - dC;
-  const double tA = fma((13.0 / 12.0) * bA, bA, 1e-6);
-  const double tB = fma((13.0 / 12.0) * bB, bB, 1e-6);
-  const double tC = fma((13.0 / 12.0) * bC, bC, 1e-6);
-  const double hd0 = 0.5 * dB, hd1 = 0.5 * dC;
-  const double A1 = fma(0.5, bA, dB), A2 = hd0 + hd1, A3 = fma(0.5, bC, -dC);
-  const double e1 = fma(A1, A1, tA), e2 = fma(A2, A2, tB), e3 = fma(A3, A3, tC);
+// With the first differences around f0, dA = f-1 - f-2, dB = f0 - f-1, dC =
+// f+1 - f0, dD = f+2 - f+1, the smoothness indicators of WENO5_JS.py:17-33 are
+// quadratic forms that complete to
+//   IS_1 = 4/3 [(dA - 11/8 dB)^2 + 39/64 dB^2]
+//   IS_2 = 4/3 [(dB -  5/8 dC)^2 + 39/64 dC^2]
+//   IS_3 = 4/3 [(dD - 11/8 dC)^2 + 39/64 dC^2]
+// (the constants are exact in binary), and the candidates are
+//   q_1 - f0 = (5 dB - 2 dA)/6, q_2 - f0 = (dB + 2 dC)/6, q_3 - f0 = (4 dC - dD)/6.
+// So one square per difference, t(d) = 39/64 d^2 + eps', serves two
+// indicators (three along a line), the common factor 4/3 goes into eps' = 3/4
+// eps, and the weights' 1 : 6 : 3 into the candidates:
+//   value = f0 + [a_1 (5/2 dB - dA) + a_2 (3 dB + 6 dC) + a_3 (6 dC - 3/2 dD)] /
+//           [3 (a_1 + 6 a_2 + 3 a_3)],   a_k = 1 / e_k^2,  e_k = 3/4 (eps + IS_k).
+// A right-biased value is the same with the stencil reversed.
+constexpr double kWenoEps = 0.75e-6;
+
+// The FP64 Lax-Friedrichs kernels hold their split fluxes scaled by 2^-20
+// (exact, undone in the divergence), which centres e_k^8 in FP64's range.
+template <typename W>
+struct LfScale { static constexpr double value = 1.0 / 1048576.0; };
+template <>
+struct LfScale<float> { static constexpr double value = 1.0; };
+constexpr double kLfEps = kWenoEps * LfScale<double>::value * LfScale<double>::value;
+
+// Three times the numerator and the denominator above with a_k = e_i^2 e_j^2 (the
+// same ratio), so the weights take no reciprocal.
+__host__ __device__ __forceinline__ void weno5_parts(double dA, double dB, double dC, double dD,
+                                                     double eps, double& num, double& den) {
+  const double tB = fma((39.0 / 64.0) * dB, dB, eps), tC = fma((39.0 / 64.0) * dC, dC, eps);
+  const double m1 = fma(-1.375, dB, dA), m2 = fma(-0.625, dC, dB), m3 = fma(-1.375, dC, dD);
+  const double e1 = fma(m1, m1, tB), e2 = fma(m2, m2, tC), e3 = fma(m3, m3, tC);
   const double s1 = e1 * e1, s2 = e2 * e2, s3 = e3 * e3;
-  const double P1 = 0.1 * (s2 * s3), P2 = 0.6 * (s1 * s3), P3 = 0.3 * (s1 * s2);
-  const double c1 = fma(1.0 / 3.0, bA, hd0);
-  const double c2 = fma(-1.0 / 6.0, bB, hd1);
-  const double c3 = fma(-1.0 / 6.0, bC, hd1);
-  return fma(fma(P1, c1, fma(P2, c2, P3 * c3)), rcp(P1 + P2 + P3), f0);
+  const double P1 = s2 * s3, P2 = s1 * s3, P3 = s1 * s2;
+  const double h = 6.0 * dC;
+  const double c1 = fma(2.5, dB, -dA), c2 = fma(3.0, dB, h), c3 = fma(-1.5, dD, h);
+  num = fma(P1, c1, fma(P2, c2, P3 * c3));
+  den = fma(6.0, P2, fma(3.0, P3, P1));
 }
 
-// FP32 form for the mixed-precision step: the FP64 form's differences and
-// candidates, with the weights normalised by the smallest e_k = eps + IS_k,
+// FP64 face value: 35 operations and one reciprocal.
+__host__ __device__ __forceinline__ double weno5(double fm2, double fm1, double f0,
+                                                 double fp1, double fp2) {
+  double num, den;
+  weno5_parts(fm1 - fm2, f0 - fm1, fp1 - f0, fp2 - fp1, kWenoEps, num, den);
+  return fma(num * (1.0 / 3.0), rcp(den), f0);
+}
+
+// FP64 face flux of the Lax-Friedrichs split: left-biased value of H+ (p0..p4)
+// plus right-biased value of H- (m1..m5), both scaled by LfScale.  The two
+// quotients are taken over one reciprocal (e_k^8 stays within FP64 for jumps of
+// up to 1e24): 67 operations and one reciprocal, 87 and two as separate values
+// in the b^2 form.
+__host__ __device__ __forceinline__ double weno5_lf(double p0, double p1, double p2, double p3,
+                                                    double p4, double m1, double m2, double m3,
+                                                    double m4, double m5) {
+  double nL, dL, nR, dR;
+  weno5_parts(p1 - p0, p2 - p1, p3 - p2, p4 - p3, kLfEps, nL, dL);
+  weno5_parts(m4 - m5, m3 - m4, m2 - m3, m1 - m2, kLfEps, nR, dR);
+  return fma(fma(nL, dR, nR * dL) * (1.0 / 3.0), rcp(dL * dR), p2 + m3);
+}
+
+// FP32 form for the mixed-precision step: first and second
+// differences b around f0 (IS_1 = (b_-1/2 + d0)^2 + 13/12 b_-1^2 and alike),
+// with the weights normalised by the smallest e_k = eps + IS_k,
 // alpha_k = C_k (e_min / e_k)^2 (ratios <= 1, the smallest weight's ratio 1).
 // e_k itself is never squared: in SI units the split energy flux jumps by
 // ~1e11 across a detonation front, so e_k reaches ~1e23 and e_k^2 would
@@ -111,6 +144,13 @@ __host__ __device__ __forceinline__ void weno5_run(const float* p, int s, float*
     dB = dC; dC = dD;
     bA = bB; tA = tB; bB = bC; tB = tC;
   }
+}
+
+// FP32 face flux of the Lax-Friedrichs split, unscaled.
+__host__ __device__ __forceinline__ float weno5_lf(float p0, float p1, float p2, float p3,
+                                                   float p4, float m1, float m2, float m3,
+                                                   float m4, float m5) {
+  return weno5(p0, p1, p2, p3, p4) + weno5(m5, m4, m3, m2, m1);
 }
 
 }  // namespace jh
