@@ -296,8 +296,8 @@ int jh_health(jh_ctx* ctx, unsigned int* flags);
 
 /* ---------------------------------------------------------------- batches
  * Many independent cases of uneven grid sizes advanced together: one launch
- * per kernel kind covers every case (the stage kernel is persistent over the
- * tile list of all cases), and jh_batch_advance can capture its launch
+ * per kernel kind covers every case (the stage kernel has a block per tile of
+ * all cases), and jh_batch_advance can capture its launch
  * sequence in a HIP graph and replay it.  Each case evolves exactly as
  * jh_advance would advance it alone (bit-identical results).  The reference
  * batches same-size blocks with jax.vmap over advance_one_step

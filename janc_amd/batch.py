@@ -3,8 +3,7 @@
 ``BatchSimulator`` takes one reference-style simulation_config per case (the
 same dict ``Simulator`` takes), binds one device state per case and advances
 all of them with the batched kernels of ``jh_batch_*``: one launch per kernel
-kind for every case, the stage kernel persistent over the tile list of all
-cases, and optionally the whole multi-step launch sequence captured in a HIP
+kind for every case, the stage kernel one block per tile of all cases, and optionally the whole multi-step launch sequence captured in a HIP
 graph and replayed.  Every case evolves bit-identically to advancing it alone
 with ``Simulator.advance``.
 

@@ -839,7 +839,6 @@ struct jh_batch {
   int* off = nullptr;                 // device block tables
   std::vector<int> h_off;
   int t_stage[kTileVariants] = {}, t_bc = 0, t_red = 0, t_chem = 0;   // table starts in off
-  int persist[kTileVariants] = {};    // persistent grid of each stage variant
   int tile = 0;
   std::vector<void*> U, aux;
   bool bound = false;
@@ -923,48 +922,22 @@ int upload_desc(jh_batch* b) {
   return JH_OK;
 }
 
-template <typename Real, int TX, int WPE>
-int persistent_grid(jh_batch* b, int v, int cus) {
-  int per_cu = 0;
-  BHIP_TRY(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                  &per_cu, stage_batch_kernel<Real, TX, WPE>, Tile<TX>::NT, 0));
-  if (per_cu < 1) per_cu = 1;
-  int g = (per_cu * cus) & ~7;
-  if (g < 8) g = 8;
-  b->persist[v] = g;
-  return JH_OK;
-}
-
-template <typename Real>
-int setup_grids(jh_batch* b) {
-  int dev = 0, cus = 0;
-  BHIP_TRY(b, hipGetDevice(&dev));
-  BHIP_TRY(b, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  int rc = JH_OK;
-#define JH_GRID(V, TX, WPE) \
-  if (!rc) rc = persistent_grid<Real, TX, WPE>(b, V, cus);
-  JH_TILE_VARIANTS(JH_GRID)
-#undef JH_GRID
-  return rc;
-}
-
 template <typename Real>
 void launch_stage_batch(jh_batch* b, hipStream_t st, int stage, int parity, double dt,
                         double cfl) {
   const auto* d = static_cast<const CaseDesc<Real>*>(b->desc);
   const int v = b->tile;
-  const int total = b->h_off[b->t_stage[v] + b->ncase];
-  const int g = std::min(b->persist[v], total);
+  const int g = b->h_off[b->t_stage[v] + b->ncase];
   const int* off = b->off + b->t_stage[v];
   switch (v) {
 #define JH_LAUNCH(V, TX, WPE)                                                           \
     case V:                                                                             \
       if (b->mirror)                                                                    \
         stage_batch_kernel<Real, TX, WPE, true><<<g, Tile<TX>::NT, 0, st>>>(            \
-            d, off, b->ncase, stage, parity, dt, cfl);                                  \
+            d, off, b->mc, b->ncase, stage, parity, dt, cfl);                           \
       else                                                                              \
         stage_batch_kernel<Real, TX, WPE><<<g, Tile<TX>::NT, 0, st>>>(                  \
-            d, off, b->ncase, stage, parity, dt, cfl);                                  \
+            d, off, b->mc, b->ncase, stage, parity, dt, cfl);                           \
       break;
     JH_TILE_VARIANTS(JH_LAUNCH)
 #undef JH_LAUNCH
@@ -982,19 +955,19 @@ int batch_enqueue(jh_batch* b, hipStream_t st, double dt, double cfl, int nsteps
   const int n_red = b->h_off[b->t_red + nc], n_bc = b->h_off[b->t_bc + nc];
   const int n_chem = b->h_off[b->t_chem + nc];
   reset_batch_kernel<Real><<<(nc + 63) / 64, 64, 0, st>>>(d, nc, 0);
-  reduce_batch_kernel<Real><<<n_red, 256, 0, st>>>(d, b->off + b->t_red, nc, 0, dt, cfl);
+  reduce_batch_kernel<Real><<<n_red, 256, 0, st>>>(d, b->off + b->t_red, b->mc, nc, 0, dt, cfl);
   for (int s = 0; s < nsteps; ++s) {
     const int parity = s & 1;
     for (int stage = 0; stage < 3; ++stage) {
       // copy-kind sides only: the stage kernel reads the halo from the
       // source cells and zeroes the other parity's slots at stage 0
       if (!b->mirror)
-        bc_batch_kernel<Real><<<n_bc, kBcThreads, 0, st>>>(d, b->off + b->t_bc, nc, stage, parity,
-                                                           dt, cfl);
+        bc_batch_kernel<Real><<<n_bc, kBcThreads, 0, st>>>(d, b->off + b->t_bc, b->mc, nc, stage,
+                                                           parity, dt, cfl);
       launch_stage_batch<Real>(b, st, stage, parity, dt, cfl);
     }
-    chem_batch_kernel<Real><<<n_chem, 256, 0, st>>>(d, b->off + b->t_chem, nc, parity, dt, cfl,
-                                                     hist, nsteps, s);
+    chem_batch_kernel<Real><<<n_chem, 256, 0, st>>>(d, b->off + b->t_chem, b->mc, nc, parity, dt,
+                                                     cfl, hist, nsteps, s);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return bfail(b, JH_ERR_HIP, std::string("batch kernels: ") +
@@ -1773,8 +1746,7 @@ int jh_batch_create(int ncase, const int* nx, const int* ny, const double* dx, c
     jh_batch_destroy(b);
     return JH_ERR_HIP;
   }
-  int rc = precision == JH_PREC_FP64 ? setup_grids<double>(b) : setup_grids<float>(b);
-  if (!rc) rc = precision == JH_PREC_FP64 ? upload_desc<double>(b) : upload_desc<float>(b);
+  const int rc = precision == JH_PREC_FP64 ? upload_desc<double>(b) : upload_desc<float>(b);
   if (rc) {
     g_batch_err = b->err;
     jh_batch_destroy(b);
