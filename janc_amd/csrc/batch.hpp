@@ -48,7 +48,7 @@ __device__ __forceinline__ T* device_ptr(T* p) {
 
 // A case's arguments.  The mechanism is the kernel's own argument, the same for
 // every case, so its constants are scalar loads as in the single-case kernels.
-// 64 mixed cases of 7.0M cells in all: chemistry 1029 -> 859 us a step, stage
+// 64 mixed cases of 7.0M cells in all: chemistry 1029 -> 859 us (700 since), stage
 // kernel 939 -> 661 us a launch.
 template <typename Real>
 __device__ __forceinline__ StepArgs<Real> case_args(const CaseDesc<Real>& d,
@@ -136,17 +136,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void chem_batch_kernel(const CaseDesc<Real>* __restrict__ d, const int* __restrict__ off,
                        const MechConst* __restrict__ mc, int ncase, int parity, double dt_fixed,
                        double cfl, double* dt_hist, int hist_len, int s) {
-  __shared__ double red[4];
-  __shared__ unsigned long long redb[4];
+  __shared__ unsigned long long red[12];
   const int k = find_case(off, ncase, blockIdx.x);
   const CaseDesc<Real>& cd = d[k];
   const StepArgs<Real> a = case_args(cd, mc, parity, dt_fixed, cfl);
-  __shared__ unsigned long long redg[kGridSlotsChem * 4];
   __shared__ MixTables mix;
   __shared__ GibbsTables gt;
   chem_body<Real, CHEM_STEP>(a, device_ptr(cd.U), device_ptr(cd.aux), nullptr,
                              dt_hist ? dt_hist + (size_t)k * hist_len + s : nullptr,
-                             blockIdx.x - off[k], red, redb, redg, mix, gt);
+                             blockIdx.x - off[k], red, nullptr, mix, gt);
 }
 
 }  // namespace jh

@@ -237,8 +237,8 @@ void blocks_chem_kernel(StepArgs<Real> a, long long bs, Real* B, int n_blk) {
   __shared__ MixTables mix;
   __shared__ GibbsTables gt;
   chem_body<Real, CHEM_STEP, false, false, true>(a, B, B + (size_t)NU * a.nx * a.ny, nullptr,
-                                                 nullptr, blockIdx.x, nullptr, nullptr, nullptr,
-                                                 mix, gt, bs, n_blk);
+                                                 nullptr, blockIdx.x, nullptr, nullptr, mix, gt, bs,
+                                                 n_blk);
 }
 
 // Ghost refill of same-size blocks tiling one uniform level: out[b][v][p]

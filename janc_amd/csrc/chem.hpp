@@ -102,9 +102,10 @@ __host__ __device__ __forceinline__ bool lu_solve(double (&A)[N][N], double (&b)
 
 // Increment of rho*Y_k for the active species (detailed_reaction, :183-193).
 // ld.rho(), ld(k): the state's rho and rho*Y_k for the NS-1 transported
-// species (register values, or loads from the state: they are read again
-// after the solve, behind a compiler barrier, so the state is not held in
-// registers across the Jacobian and its factorisation); gt: the Gibbs tables (c
+// species.  A kernel's state is not held in registers across the Jacobian:
+// ld.again() reads it a second time, ahead of the factorisation, whose time
+// covers the reads; after it rho() and ld(k) are those values.  gt: the Gibbs
+// tables (c
 // itself, or its copy in LDS); JT: the Jacobian's storage type (float in the
 // mixed-precision form: assembled in FP32 from FP64 terms, factorised and
 // solved in FP64).  Returns lu_solve's pivot check.  clip (optional): bit k
@@ -114,7 +115,7 @@ __host__ __device__ __forceinline__ bool lu_solve(double (&A)[N][N], double (&b)
 // state on the branches of another).
 template <typename JT = double, typename GTab, typename LoadRY>
 __host__ __device__ __forceinline__ bool chem_increment_ld(const MechConst& c, const GTab& gt,
-                                                           const LoadRY& ld, double T, double dt,
+                                                           LoadRY& ld, double T, double dt,
                                                            double (&drhoY)[JH_NA],
                                                            unsigned int* clip = nullptr,
                                                            const unsigned int* branches = nullptr) {
@@ -153,10 +154,8 @@ __host__ __device__ __forceinline__ bool chem_increment_ld(const MechConst& c, c
 #pragma unroll
     for (int n = 0; n < JH_NA; ++n) A[k][n] = ((k == n) ? idt : 0.0) - (double)J[k][n];
   }
+  ld.again();
   const bool ok = lu_solve<JH_NA>(A, w);
-#if defined(__HIP_DEVICE_COMPILE__)
-  __asm__ volatile("" ::: "memory");   // ld below reloads
-#endif
   const double rho = ld.rho(), irho = rcp(rho);
   unsigned int cm = 0u;
 #pragma unroll
@@ -183,6 +182,7 @@ struct RegState {
   const double (&y)[JH_NS - 1];
   __host__ __device__ double rho() const { return r; }
   __host__ __device__ double operator()(int k) const { return y[k]; }
+  __host__ __device__ void again() {}
 };
 
 template <typename JT = double, typename GTab>
@@ -193,7 +193,8 @@ __host__ __device__ __forceinline__ bool chem_increment(const MechConst& c, cons
                                                         double (&drhoY)[JH_NA],
                                                         unsigned int* clip = nullptr,
                                                         const unsigned int* branches = nullptr) {
-  return chem_increment_ld<JT>(c, gt, RegState{rho, rhoY_in}, T, dt, drhoY, clip, branches);
+  RegState ld{rho, rhoY_in};
+  return chem_increment_ld<JT>(c, gt, ld, T, dt, drhoY, clip, branches);
 }
 
 __host__ __device__ __forceinline__ bool chem_increment(const MechConst& c, double rho,
