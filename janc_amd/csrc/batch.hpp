@@ -124,7 +124,7 @@ void stage_batch_kernel(const CaseDesc<Real>* __restrict__ d, const int* __restr
   const Real* As = stage == 0 ? cd.aux : stage == 1 ? cd.A1 : cd.A2;
   Real* Uo = stage == 0 ? cd.U1 : stage == 1 ? cd.U2 : cd.U;
   Real* Ao = stage == 0 ? cd.A1 : stage == 1 ? cd.A2 : cd.aux;
-  stage_body<Real, MODE_RK, TX, RECON_WENO5, SPLIT_LF, Real, false, false, MIRROR>(
+  stage_body<Real, MODE_RK, TX, RECON_WENO5, SPLIT_LF, Real, false, MIRROR>(
       a, stage, device_ptr(Us), device_ptr(As), device_ptr(cd.U), device_ptr(Uo), device_ptr(Ao),
       t - off[k], L);
 }

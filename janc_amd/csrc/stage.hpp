@@ -115,6 +115,14 @@ __device__ __forceinline__ void block_max_bits_multi(unsigned long long (&v)[K],
   }
 }
 
+// A value every lane of the wave holds, in scalar registers.
+__device__ __forceinline__ double wave_uniform(double v) {
+  const unsigned long long b = dbits(v);
+  const unsigned int lo = __builtin_amdgcn_readfirstlane((unsigned int)b);
+  const unsigned int hi = __builtin_amdgcn_readfirstlane((unsigned int)(b >> 32));
+  return bitsd(((unsigned long long)hi << 32) | lo);
+}
+
 // Maximum over the wave of a value's bits, in lane 63: DPP moves (rows of 16, then
 // row to row), no LDS traffic.
 template <int CTRL, int ROWS>
@@ -238,33 +246,49 @@ struct Prim {
   W rho, u, v, p, a, g;       // g: gamma from aux (set with a)
 };
 
-template <typename W, bool WITH_A, typename Real>
-__device__ __forceinline__ Prim<W> cell_prim(const MechConst& c, const Real* __restrict__ Up,
-                                             const Real* __restrict__ ap, int stride) {
+// ld(v): plane v of the cell, v = 0..11 the conserved variables, 12 gamma, 13 T.
+template <typename W, bool WITH_A, typename Load>
+__device__ __forceinline__ Prim<W> cell_prim_ld(const MechConst& c, const Load& ld) {
   Prim<W> q;
-  q.rho = (W)Up[0];
+  q.rho = (W)ld(0);
   const W ir = rcp(q.rho);
-  q.u = (W)Up[stride] * ir;
-  q.v = (W)Up[2 * stride] * ir;
+  q.u = (W)ld(1) * ir;
+  q.v = (W)ld(2) * ir;
   W sum = (W)0, R = (W)0;
   W Y[JH_NS];
 #pragma unroll
   for (int k = 0; k < JH_NS - 1; ++k) {
-    Y[k] = (W)Up[(4 + k) * stride] * ir;
+    Y[k] = (W)ld(4 + k) * ir;
     sum += Y[k];
   }
   Y[JH_NS - 1] = (W)1 - sum;
 #pragma unroll
   for (int k = 0; k < JH_NS; ++k) R += (W)c.R[k] * Y[k];
-  const W T = (W)ap[stride];
+  const W T = (W)ld(13);
   q.p = (q.rho * R * T);
   q.a = (W)0;
   q.g = (W)0;
   if (WITH_A) {
-    q.g = (W)ap[0];
+    q.g = (W)ld(12);
     q.a = sqrt(q.g * q.p * ir);
   }
   return q;
+}
+
+template <typename W, bool WITH_A, typename Real>
+__device__ __forceinline__ Prim<W> cell_prim(const MechConst& c, const Real* __restrict__ Up,
+                                             const Real* __restrict__ ap, int stride) {
+  return cell_prim_ld<W, WITH_A>(c, [&](int v) { return v < 12 ? Up[v * stride]
+                                                               : ap[(v - 12) * stride]; });
+}
+
+// Element at byte offset off of a plane whose address is wave-uniform: the plane
+// stays in scalar registers and the cell is one 32-bit offset, so an access costs
+// no vector address arithmetic.
+template <typename Real>
+__device__ __forceinline__ Real& at(Real* plane, unsigned int off) {
+  using Byte = std::conditional_t<std::is_const<Real>::value, const char, char>;
+  return *reinterpret_cast<Real*>(reinterpret_cast<Byte*>(plane) + off);
 }
 
 // ------------------------------------------------------------- arguments
@@ -973,6 +997,44 @@ __device__ __forceinline__ W face_sum(const W* p, const W* m, int s) {
          recon_R<RECON, W>(m[s], m[2 * s], m[3 * s], m[4 * s], m[5 * s]);
 }
 
+// The stencils of one face: H+ from p, H- from m, five values each, s apart.
+template <typename W>
+struct FaceLine {
+  const W* p;
+  const W* m;
+  int s;
+};
+
+// Fluxes (weno5_lf, bit for bit) of N faces of the FP64 Lax-Friedrichs split, one
+// after another: the reads of a face's H- run while its H+ is worked on, those of
+// the next face's H+ while its H- is.  The FP64 kernel is bound by that latency and
+// by FP64 issue at four waves per SIMD (two blocks' LDS): a loop over single faces
+// with a division for each one's place took 271 us a stage of the 4000 x 400 annulus,
+// this with scalar addresses 259; wider windows (pairs, runs of four) save reads and
+// operations and lose more to spills or to a third of the waves.
+template <int N>
+__device__ __forceinline__ void face_chain(const FaceLine<double> (&l)[N], double* const (&out)[N]) {
+  double p[5], m[5];
+#pragma unroll
+  for (int j = 0; j < 5; ++j) p[j] = l[0].p[j * l[0].s];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    double nL, dL, nR, dR;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) m[j] = l[i].m[j * l[i].s];
+    __builtin_amdgcn_sched_barrier(0);
+    weno5_parts(p[1] - p[0], p[2] - p[1], p[3] - p[2], p[4] - p[3], kLfEps, nL, dL);
+    const double p2 = p[2];
+    if (i + 1 < N) {
+#pragma unroll
+      for (int j = 0; j < 5; ++j) p[j] = l[i + 1].p[j * l[i + 1].s];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    weno5_parts(m[3] - m[4], m[2] - m[3], m[1] - m[2], m[0] - m[1], kLfEps, nR, dR);
+    *out[i] = fma(fma(nL, dR, nR * dL) * (1.0 / 3.0), rcp(dL * dR), p2 + m[2]);
+  }
+}
+
 // One SSP-RK3 stage (TVD_RK3.py:5-12) for a 64 x TX tile:
 //   rhs = dt * -(dF/dx + dG/dy)   (set_simulator.py:44-47, flux.py:56-68)
 //   stage 0: U1 = U + rhs; stage 1: U2 = 3/4 U + 1/4 (U1 + rhs);
@@ -996,7 +1058,7 @@ struct StageLds {
   Real Hyp[TX][TY + 6], Hym[TX][TY + 6];
   Real Fx[TX + 1][TY];
   Real Fy[TX][TY + 1];
-  double red[Tile<TX>::NW];
+  unsigned long long red[2 * Tile<TX>::NW];
   MixTables mix;              // NASA-7 tables for the Halley epilogue
 };
 
@@ -1005,11 +1067,10 @@ struct StageLds {
 // W the arithmetic type of the split fluxes, reconstructions, divergence and
 // RK combine (Real, the storage type, unless stated); GRID the grid-wide
 // temperature-solve stop (StepArgs::hside set), compiled separately so the
-// per-cell kernels keep their register budget; PAD the state planes are one
-// AMR block with its own ghost layers ((nx + 6) x (ny + 6), no ghost strips,
-// no next-stage maxima: the next stage's ghosts come from the caller).
+// per-cell kernels keep their register budget; MIRROR the halo is read from the
+// source cells of copy-kind sides (locate_src).
 template <typename Real, int MODE, int TX, int RECON = RECON_WENO5, int SPLIT = SPLIT_LF,
-          typename W = Real, bool GRID = false, bool PAD = false, bool MIRROR = false>
+          typename W = Real, bool GRID = false, bool MIRROR = false>
 __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
                                            const Real* __restrict__ Us,
                                            const Real* __restrict__ auxs, const Real* Un,
@@ -1024,16 +1085,16 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
   auto& sHym = L.Hym;
   auto& sFx = L.Fx;
   auto& sFy = L.Fy;
-  double* red = L.red;
   (void)NW;
-  // face runs for the FP32 WENO5 (the FP64 form's carried differences would
-  // push the kernel past its register budget)
+  // face runs, whose neighbouring faces share differences (weno.hpp).  FP32 only:
+  // an FP64 run's carried values cost the kernel a wave per SIMD, and two steps of
+  // 4000 x 500 took 2200 us with it where single faces took 2180
   constexpr bool kRuns = RECON == RECON_WENO5 && std::is_same<W, float>::value;
   static_assert(!kRuns || (TX % 4 == 0 && TX <= 64), "face runs need TX a multiple of 4");
 
   const MechConst& c = *a.mc;
   if (MODE != MODE_RHS) load_mix_tables(c, L.mix);   // read after the phase barriers
-  const int nx = a.nx, ny = a.ny, n = PAD ? (nx + 6) * (ny + 6) : nx * ny;
+  const int nx = a.nx, ny = a.ny, n = nx * ny;
   // the wave index through readfirstlane: the tile rows, slots and face
   // runs derived from it are wave-uniform to the compiler (scalar registers
   // and branches)
@@ -1046,18 +1107,26 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
   const int tiles_y = (ny + TY - 1) / TY;
   const int x0 = (tile / tiles_y) * TX;
   const int y0 = (tile % tiles_y) * TY;
-  const double dt = step_dt(a);
+  // FP64 holds the block's constants in scalar registers and addresses a cell by
+  // scalar plane and byte offset (at).  FP32 has registers to spare and measured 1 %
+  // slower with either (mixed tube of 8000 x 500: 6430 -> 6490 us for four steps).
+  constexpr bool kScalar = sizeof(W) == 8;
+  const auto uniform = [](auto v) {
+    if constexpr (kScalar) return wave_uniform(v);
+    else return v;
+  };
+  const double dt = uniform(step_dt(a));
   // Lax-Friedrichs split fluxes with WENO5 are held scaled (LfScale), undone in
   // the divergence
   constexpr double sc =
       RECON == RECON_WENO5 && SPLIT == SPLIT_LF ? LfScale<W>::value : 1.0;
   constexpr W hs = (W)(0.5 * sc);
-  const double idx = 1.0 / sc / a.dx, idy = 1.0 / sc / a.dy;
+  const double idx = uniform(1.0 / sc / a.dx), idy = uniform(1.0 / sc / a.dy);
   const W ax = (W)(Real)bitsd(a.sc->amax[a.parity][stage][0]);
   const W ay = (W)(Real)bitsd(a.sc->amax[a.parity][stage][1]);
   // H+- = (F +- alpha U) / 2 as fma(+-alpha/2, U, F/2): halving is exact, so
   // this is the same value with one operation fewer per pair
-  const W hax = hs * ax, hay = hs * ay;
+  const W hax = uniform(hs * ax), hay = uniform(hs * ay);
 
   int rrow[NSL], rcol[NSL];       // LDS coordinates: x-region row / y-region col
   int gxs[NSL], gys[NSL];
@@ -1087,6 +1156,13 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
     gys[s] = y0 - 3 + col;
   }
   CellRef<Real> ref[NSL];
+  unsigned int off[NSL];          // byte offset of the slot's cell in a plane
+  constexpr bool kOff = MIRROR && kScalar;
+  // plane v of slot s
+  const auto ld = [&](int s, int v) -> Real {
+    if constexpr (kOff) return at(Us + (size_t)v * n, off[s]);
+    else return ref[s].u[v * ref[s].stride];
+  };
   Prim<W> q[NSL];
   Real nxt[NSL];
   // bits 2s, 2s + 1: slot s is a ghost whose rho u, rho v its side negates
@@ -1095,16 +1171,21 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
 #pragma unroll
   for (int s = 0; s < NSL; ++s) {
     unsigned int f = 0u;
-    if constexpr (PAD) ref[s] = locate_padded<Real>(a, Us, auxs, gxs[s], gys[s]);
-    else if constexpr (MIRROR) ref[s] = locate_src<Real>(a, Us, auxs, gxs[s], gys[s], f);
+    if constexpr (MIRROR) ref[s] = locate_src<Real>(a, Us, auxs, gxs[s], gys[s], f);
     else ref[s] = locate<Real>(a, Us, auxs, gxs[s], gys[s]);
     if (!has[s]) ref[s].ok = false;
+    if constexpr (kOff) off[s] = (unsigned int)((ref[s].u - Us) * sizeof(Real));
     if (ref[s].ok) {
-      q[s] = cell_prim<W, SPLIT == SPLIT_SW, Real>(c, ref[s].u, ref[s].x, ref[s].stride);
+      if constexpr (kOff)
+        q[s] = cell_prim_ld<W, false>(c, [&](int v) {
+          return v < NU ? at(Us + (size_t)v * n, off[s]) : at(auxs + (size_t)(v - NU) * n, off[s]);
+        });
+      else
+        q[s] = cell_prim<W, SPLIT == SPLIT_SW, Real>(c, ref[s].u, ref[s].x, ref[s].stride);
       if (f & 1u) q[s].u = -q[s].u;
       if (f & 2u) q[s].v = -q[s].v;
       flips |= f << (2 * s);
-      nxt[s] = ref[s].u[0];
+      nxt[s] = ld(s, 0);
     } else {
       q[s].rho = (W)1; q[s].u = (W)0; q[s].v = (W)0; q[s].p = (W)0; q[s].a = (W)0;
       q[s].g = (W)1;
@@ -1116,8 +1197,14 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     own[s] = gxs[s] < nx && gys[s] < ny;
-    oidx[s] = PAD ? (gxs[s] + 3) * (ny + 6) + gys[s] + 3 : gxs[s] * ny + gys[s];
+    oidx[s] = gxs[s] * ny + gys[s];
   }
+  const auto own_at = [&](auto* base, int v, int s) -> auto& {   // own cell s of plane v
+    if constexpr (kScalar)
+      return at(base + (size_t)v * n, (unsigned int)oidx[s] * (unsigned int)sizeof(Real));
+    else
+      return base[v * n + oidx[s]];
+  };
 
   // One conserved variable; CLS = min(cv, 4) selects the physical flux
   // (and the Steger-Warming split) at compile time, so phase 1 carries no
@@ -1172,23 +1259,22 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
     if (cv + 1 < NU) {
 #pragma unroll
       for (int s = 0; s < NSL; ++s)
-        if (ref[s].ok) nxt[s] = ref[s].u[(cv + 1) * ref[s].stride];
+        if (ref[s].ok) nxt[s] = ld(s, cv + 1);
     }
     W u0n[2] = {(W)0, (W)0};
     if (MODE != MODE_RHS && stage != 0) {
 #pragma unroll
       for (int s = 0; s < 2; ++s)
-        if (own[s]) u0n[s] = (W)Un[cv * n + oidx[s]];
+        if (own[s]) u0n[s] = (W)own_at(Un, cv, s);
     }
     // ---- phase 2: face reconstructions ----
     if constexpr (kRuns) {
-      // FP32 WENO5: runs of consecutive faces (weno5_run).  The first half
-      // of the block takes the x faces: lane = column, wave = run (TX / 4
-      // runs of four per column, the last a run of five through face row
-      // TX); its first wave also takes the y faces of column 64 (lane =
-      // row), so no y wave runs a single-face pass for a few of its lanes.
-      // The second half the y faces 0..63: 16 runs of four per row, run =
-      // u % 16, row = u / 16.
+      // runs of consecutive faces.  The first half of the block takes the x
+      // faces: lane = column, wave = run (TX / 4 runs of four per column, the
+      // last a run of five through face row TX); its first wave also takes the y
+      // faces of column 64 (lane = row), so no y wave runs a single-face pass for
+      // a few of its lanes.  The second half the y faces 0..63: 16 runs of four
+      // per row, run = u % 16, row = u / 16.
       constexpr int NXT = NT / 2;
       static_assert(NXT % 64 == 0, "the x-face half of the block is whole waves");
       if (w < NXT / 64) {
@@ -1212,6 +1298,18 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
         weno5_run<4, false, false>(&sHyp[row][fc0], 1, &sFy[row][fc0], 1);
         weno5_run<4, true, true>(&sHym[row][fc0 + 1], 1, &sFy[row][fc0], 1);
       }
+    } else if constexpr (RECON == RECON_WENO5 && SPLIT == SPLIT_LF) {
+      // FP64: a thread's two x faces and two y faces (rows w and w + NW, column
+      // ly), then face row TX by the last wave and face column 64 by the first.
+      // Reads of one side run while the other side's weights are formed.
+      const auto xp = [&](int r) { return FaceLine<W>{&sHxp[r][ly], &sHxm[r + 1][ly], TY}; };
+      const auto yp = [&](int r) { return FaceLine<W>{&sHyp[r][ly], &sHym[r][ly + 1], 1}; };
+      const FaceLine<W> line[4] = {xp(w), xp(w + NW), yp(w), yp(w + NW)};
+      W* const out[4] = {&sFx[w][ly], &sFx[w + NW][ly], &sFy[w][ly], &sFy[w + NW][ly]};
+      face_chain<4>(line, out);
+      if (w == NW - 1) sFx[TX][ly] = face_sum<RECON, SPLIT, W>(&sHxp[TX][ly], &sHxm[TX][ly], TY);
+      if (w == 0 && ly < TX)
+        sFy[ly][TY] = face_sum<RECON, SPLIT, W>(&sHyp[ly][TY], &sHym[ly][TY], 1);
     } else
     for (int it = t; it < NXF + NYF; it += NT) {
       if (it < NXF) {
@@ -1246,7 +1344,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
         if (stage == 1) un = (3.0 / 4.0) * u0 + (1.0 / 4.0) * (uc + rhs);
         else un = (1.0 / 3.0) * u0 + (2.0 / 3.0) * (uc + rhs);
       }
-      if (own[s]) Uo[cv * n + oidx[s]] = (Real)un;
+      if (own[s]) own_at(Uo, cv, s) = (Real)un;
     }
     // (no explicit drain of the memory counters here: with the loop
     // specialised per variable class the compiler's own waits are as good,
@@ -1272,32 +1370,34 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if (!own[s]) continue;
-    const Real* un = Uo + oidx[s];
+    Real un[NU];
+#pragma unroll
+    for (int k = 0; k < NU; ++k) un[k] = own_at(Uo, k, s);
     const double rho = (double)un[0], ir = rcp(rho);
-    const double u = (double)un[n] * ir, v = (double)un[2 * n] * ir;
-    const double e = (double)un[3 * n] * ir - 0.5 * (u * u + v * v);
+    const double u = (double)un[1] * ir, v = (double)un[2] * ir;
+    const double e = (double)un[3] * ir - 0.5 * (u * u + v * v);
     double Y[JH_NS];
 #pragma unroll
-    for (int k = 0; k < JH_NS - 1; ++k) Y[k] = (double)un[(4 + k) * n] * ir;
+    for (int k = 0; k < JH_NS - 1; ++k) Y[k] = (double)un[4 + k] * ir;
     const double R = fill_Y_get_R(c, Y);
-    double T = (double)auxs[n + oidx[s]];
+    double T = (double)own_at(auxs, 1, s);
     double gamma;
     HalleyMore hm{0, 0.0, 0.0, true, true};
     bool conv;
     if constexpr (grid) {
       conv = halley_T<MixTables, true>(L.mix, Y, R, e, T, gamma, &hm);
-      a.hside[oidx[s]] = (Real)hm.g1;
-      a.hside[n + oidx[s]] = (Real)hm.T1;
+      own_at(a.hside, 0, s) = (Real)hm.g1;
+      own_at(a.hside, 1, s) = (Real)hm.T1;
       a.hnit[oidx[s]] = (unsigned char)hm.n;
       if (hm.n < kHalleyMaxIter && !hm.ok1) fl |= JH_FLAG_HALLEY_REGRESS;
       gv[0] = (unsigned long long)hm.n > gv[0] ? (unsigned long long)hm.n : gv[0];
     } else {
       conv = halley_T(L.mix, Y, R, e, T, gamma);
     }
-    auxo[oidx[s]] = (Real)gamma;
-    auxo[n + oidx[s]] = (Real)T;
+    own_at(auxo, 0, s) = (Real)gamma;
+    own_at(auxo, 1, s) = (Real)T;
     fl |= halley_flags(rho, e, R, T, gamma, conv);
-    if (!PAD && stage < 2) {
+    if (stage < 2) {
       // next stage's alpha from the stored (rounded) values
       const double gs = (double)(Real)gamma, Ts = (double)(Real)T;
       const double p = rho * R * Ts;
@@ -1321,9 +1421,9 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
     // (the reduction's first barrier)
     block_max_bits_multi<NT, kGridSlotsStage>(gv, &a.sc->gs[a.parity][stage].nstar,
                                               reinterpret_cast<unsigned long long*>(&L.Hxp[0][0]));
-  } else if (!PAD && stage < 2) {
-    block_max_atomic<NT>(mx, &a.sc->amax[a.parity][stage + 1][0], red);
-    block_max_atomic<NT>(my, &a.sc->amax[a.parity][stage + 1][1], red);
+  } else if (stage < 2) {
+    const unsigned long long m[2] = {dbits(mx), dbits(my)};
+    block_max_to<NT, 2>(m, [&](int k) { return &a.sc->amax[a.parity][stage + 1][k]; }, L.red);
   }
 }
 
@@ -1334,7 +1434,7 @@ void stage_kernel(StepArgs<Real> a, int stage, const Real* __restrict__ Us,
                   const Real* __restrict__ auxs, const Real* Un, Real* Uo,
                   Real* __restrict__ auxo) {
   __shared__ StageLds<W, TX> L;
-  stage_body<Real, MODE, TX, RECON, SPLIT, W, GRID, false, MIRROR>(a, stage, Us, auxs, Un, Uo, auxo,
+  stage_body<Real, MODE, TX, RECON, SPLIT, W, GRID, MIRROR>(a, stage, Us, auxs, Un, Uo, auxo,
                                                     xcd_tile(blockIdx.x, gridDim.x), L);
 }
 
