@@ -174,7 +174,8 @@ __device__ __forceinline__ void prim_to_U_vjp(const MechConst& c, const PrimD& q
 // grid) and dq/dv_m the WENO gradient of face f with respect to its m-th
 // stencil value.  Everything after H+-_bar (the split flux's and the
 // primitive map's VJPs) is linear in it, so the x and y contributions add:
-//   adj_prim_kernel    (rho, u, v, p) of every interior cell, for the x pass;
+//   getT_split_kernel  (ahead of the passes) also writes (rho, u, v, p) of every
+//                      interior cell, for the x pass;
 //   flux_vjp_x_kernel  H+-_bar of the x faces of every padded cell of every
 //                      interior column, swept along x in registers;
 //   flux_vjp_y_kernel  the y faces' H+-_bar, exchanged between the lanes of
@@ -184,17 +185,16 @@ __device__ __forceinline__ void prim_to_U_vjp(const MechConst& c, const PrimD& q
 // No pass uses a block barrier inside its variable loop and none keeps face
 // quantities in LDS.
 
-// x pass: one thread per (interior column, variable, side, segment of
-// kXSeg padded rows), the 64 lanes of a wave on consecutive columns.
-constexpr int kXSeg = 32;
-__host__ __device__ inline int xs_segments(int nx) { return (nx + 6 + kXSeg - 1) / kXSeg; }
+// x pass: one thread per (interior column, variable, side, segment of xseg
+// padded rows), the 64 lanes of a wave on consecutive columns.
+__host__ __device__ inline int xs_segments(int nx, int xseg) { return (nx + 6 + xseg - 1) / xseg; }
 // (variable, side) instances x groups of four tiles, one block (4 waves)
 // each; the launch rounds it up to a multiple of the 8 XCDs
-__host__ __device__ inline int xs_work_blocks(int nx, int ny) {
-  return 2 * NU * ((((ny + 63) / 64) * xs_segments(nx) + 3) / 4);
+__host__ __device__ inline int xs_work_blocks(int nx, int ny, int xseg) {
+  return 2 * NU * ((((ny + 63) / 64) * xs_segments(nx, xseg) + 3) / 4);
 }
-__host__ __device__ inline int xs_blocks(int nx, int ny) {
-  return (xs_work_blocks(nx, ny) + 7) / 8 * 8;
+__host__ __device__ inline int xs_blocks(int nx, int ny, int xseg) {
+  return (xs_work_blocks(nx, ny, xseg) + 7) / 8 * 8;
 }
 
 // y pass: a wave covers 64 consecutive padded columns of one padded row and
@@ -237,13 +237,11 @@ __device__ __forceinline__ double phys_flux_l(int cv, int dir, const PrimL& q, d
   }
 }
 
-__global__ __launch_bounds__(256) void adj_prim_kernel(AdjArgs a, const double* __restrict__ U,
-                                                       const double* __restrict__ aux,
-                                                       double* __restrict__ qb) {
-  const int n = a.nx * a.ny;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const PrimD q = prim_src(*a.mc, U, aux, n, t, 0);
+// (rho, u, v, p) of interior cell t, for the x pass.
+__device__ __forceinline__ void adj_prim_cell(const MechConst& c, const double* __restrict__ U,
+                                              const double* __restrict__ aux,
+                                              double* __restrict__ qb, int n, int t) {
+  const PrimD q = prim_src(c, U, aux, n, t, 0);
   qb[t] = q.rho;
   qb[n + t] = q.u;
   qb[2 * n + t] = q.v;
@@ -253,7 +251,7 @@ __global__ __launch_bounds__(256) void adj_prim_kernel(AdjArgs a, const double* 
 // x faces f = 0..nx of column j; the stencil of face f is padded rows
 // b .. b+4 with b = f + side, and face f's m-th gradient entry belongs to row
 // b + m (side 0) or b + 4 - m (side 1).  A thread sweeps the faces reaching
-// its rows [c0, c0 + kXSeg), holding the five stencil values and the five
+// its rows [c0, c0 + xseg), holding the five stencil values and the five
 // open row sums: row b is complete once face f = b - side is done.
 // hx[side][cv][P][j]: H+_bar (side 0) and H-_bar (side 1) of padded row P.
 // CLS = min(cv, 4) selects the physical flux and the momentum flips at
@@ -262,13 +260,14 @@ template <int CLS, int SIDE>
 __device__ __forceinline__ void xs_sweep(const AdjArgs& a, const double* __restrict__ U,
                                          const double* __restrict__ qb,
                                          const double* __restrict__ rbar, double ax,
-                                         double* __restrict__ hx, int cv, int j, int seg) {
+                                         double* __restrict__ hx, int cv, int j, int seg,
+                                         int xseg) {
   const int nx = a.nx, ny = a.ny, n = nx * ny, PX = nx + 6;
   constexpr int side = SIDE;
   const double hal = (side == 0 ? 0.5 : -0.5) * ax;
   const double dtdx = a.dt / a.dx;
-  const int c0 = seg * kXSeg, c1 = min(c0 + kXSeg, PX);
-  const int fA = max(0, c0 - 4 - side), fB = min(nx, c0 + kXSeg - 1 - side);
+  const int c0 = seg * xseg, c1 = min(c0 + xseg, PX);
+  const int fA = max(0, c0 - 4 - side), fB = min(nx, c0 + xseg - 1 - side);
   const double* Uv = U + (size_t)cv * n;
   const double* rv = rbar + (size_t)cv * n + j;
   double* out = hx + (size_t)(side * NU + cv) * PX * ny + j;
@@ -377,9 +376,9 @@ __global__ __launch_bounds__(256) void flux_vjp_x_kernel(AdjArgs a, const double
                                                          const double* __restrict__ qb,
                                                          const double* __restrict__ rbar,
                                                          const unsigned long long* alpha_bits,
-                                                         double* __restrict__ hx) {
+                                                         double* __restrict__ hx, int xseg) {
   const int nx = a.nx, ny = a.ny;
-  const int njb = (ny + 63) >> 6, nt = njb * xs_segments(nx);
+  const int njb = (ny + 63) >> 6, nt = njb * xs_segments(nx, xseg);
   // Blocks go round-robin to the 8 XCDs; logical block lb gives XCD x the
   // contiguous run lb = x * (gridDim.x / 8) + k, and consecutive logical
   // blocks are the 2 NU (variable, side) instances of one group of four
@@ -388,7 +387,7 @@ __global__ __launch_bounds__(256) void flux_vjp_x_kernel(AdjArgs a, const double
   // there by all of them.  gridDim.x is xs_blocks (a multiple of 8); the
   // logical blocks past xs_work_blocks have no work.
   const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (lb >= xs_work_blocks(nx, ny)) return;
+  if (lb >= xs_work_blocks(nx, ny, xseg)) return;
   // the wave index through readfirstlane: every quantity derived from it
   // (segment, rows, faces, loop bounds) is then wave-uniform to the compiler
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -400,16 +399,16 @@ __global__ __launch_bounds__(256) void flux_vjp_x_kernel(AdjArgs a, const double
   if (j >= ny) return;
   const double ax = bitsd(alpha_bits[0]);
   switch (2 * min(cv, 4) + side) {
-    case 0: xs_sweep<0, 0>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 1: xs_sweep<0, 1>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 2: xs_sweep<1, 0>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 3: xs_sweep<1, 1>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 4: xs_sweep<2, 0>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 5: xs_sweep<2, 1>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 6: xs_sweep<3, 0>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 7: xs_sweep<3, 1>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    case 8: xs_sweep<4, 0>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
-    default: xs_sweep<4, 1>(a, U, qb, rbar, ax, hx, cv, j, seg); break;
+    case 0: xs_sweep<0, 0>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 1: xs_sweep<0, 1>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 2: xs_sweep<1, 0>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 3: xs_sweep<1, 1>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 4: xs_sweep<2, 0>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 5: xs_sweep<2, 1>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 6: xs_sweep<3, 0>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 7: xs_sweep<3, 1>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    case 8: xs_sweep<4, 0>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
+    default: xs_sweep<4, 1>(a, U, qb, rbar, ax, hx, cv, j, seg, xseg); break;
   }
 }
 
@@ -812,20 +811,24 @@ __device__ __forceinline__ void eY_to_U(const double (&Uc)[NU], double eb,
 // Ub += VJP of aux = get_T(U) at the converged aux (gamma_bar, T_bar = ab).
 // The U cotangent that (gamma_bar, T_bar) = (ab[t], ab[n + t]) of cell t
 // sends through get_T's VJP and (e, Y)(U).
+// The tables are staged into mix while the cell is read.
 __device__ __forceinline__ void getT_vjp_cell(const MechConst& c, const double* __restrict__ U,
                                               const double* __restrict__ aux,
                                               const double* __restrict__ ab, int n, int t,
-                                              double (&Ubc)[NU]) {
+                                              MixTables& mix, double (&Ubc)[NU]) {
+  load_mix_tables(c, mix);
   double Uc[NU];
 #pragma unroll
   for (int v = 0; v < NU; ++v) Uc[v] = U[v * n + t];
+  const double T = aux[n + t], gb = ab[t], Tb = ab[n + t];
+  __syncthreads();
   const double ir = rcp(Uc[0]);
   double Y[JH_NS];
 #pragma unroll
   for (int k = 0; k < JH_NS - 1; ++k) Y[k] = Uc[4 + k] * ir;
   const double R = fill_Y_get_R(c, Y);
   double eb, Yb[JH_NS - 1];
-  getT_vjp(c, Y, R, aux[n + t], ab[t], ab[n + t], eb, Yb);
+  getT_vjp(c, mix, Y, R, T, gb, Tb, eb, Yb);
 #pragma unroll
   for (int v = 0; v < NU; ++v) Ubc[v] = 0.0;
   eY_to_U(Uc, eb, Yb, Ubc);
@@ -838,11 +841,12 @@ __global__ __launch_bounds__(256) void getT_vjp_kernel(AdjArgs a, const double* 
                                                        const double* __restrict__ ab,
                                                        const double* __restrict__ Ubar,
                                                        double* __restrict__ Ub) {
+  __shared__ MixTables mix;
   const int n = a.nx * a.ny;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
   double Ubc[NU];
-  getT_vjp_cell(*a.mc, U, aux, ab, n, t, Ubc);
+  getT_vjp_cell(*a.mc, U, aux, ab, n, min(t, n - 1), mix, Ubc);
+  if (t >= n) return;
 #pragma unroll
   for (int v = 0; v < NU; ++v) Ub[v * n + t] = Ubar[v * n + t] + Ubc[v];
 }
@@ -919,19 +923,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 // U' = ... + cr (U_s + r(U_s)), in one pass over the cells: with x = Ub +
 // get_T's VJP of ab (the value getT_vjp_kernel would store), Uacc =
 // aacc*x + bacc*Uacc (bacc = 0 overwrites), Ub = x (cr = 0) or
-// rb = Ub = cr*x, and ab zeroed.
+// rb = Ub = cr*x, and ab zeroed.  Also the primitives qb of the flux VJP's stage
+// input (Uq, Aq).  On a large grid bound by its 80 planes, on a small one by
+// latency: the NASA-7 coefficients come from LDS (as vector loads by a per-lane
+// index they were 80 of a thread's 115 reads) and the primitives had a launch of
+// their own.  16384 cells 10.3 + 3.7 -> 10.4 us, 262144 cells 33.1 + 7.2 -> 29.6 us.
 __global__ __launch_bounds__(256) void getT_split_kernel(AdjArgs a, const double* __restrict__ U,
                                                          const double* __restrict__ aux,
                                                          double aacc, double bacc, double cr,
                                                          double* __restrict__ Ub,
                                                          double* __restrict__ Uacc,
                                                          double* __restrict__ rb,
-                                                         double* __restrict__ ab) {
+                                                         double* __restrict__ ab,
+                                                         const double* __restrict__ Uq,
+                                                         const double* __restrict__ Aq,
+                                                         double* __restrict__ qb) {
+  __shared__ MixTables mix;
   const int n = a.nx * a.ny;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
   double Ubc[NU];
-  getT_vjp_cell(*a.mc, U, aux, ab, n, t, Ubc);
+  getT_vjp_cell(*a.mc, U, aux, ab, n, min(t, n - 1), mix, Ubc);
+  if (t >= n) return;
+  adj_prim_cell(*a.mc, Uq, Aq, qb, n, t);
 #pragma unroll
   for (int v = 0; v < NU; ++v) {
     const size_t i = (size_t)v * n + t;

@@ -637,14 +637,24 @@ int adj_fold(jh_ctx* c, const AdjArgs& a, AdjWork& w) {
   return JH_OK;
 }
 
-// Flux VJP of one RK stage with input (Us, As) and rhs cotangent rb; the
-// results are added into (Ut, At).
+// Rows of the x pass's segments: a segment also sweeps the 4 faces before it, so long
+// ones do the least work, until they leave SIMDs without a wave.  Reverse sweeps of 8
+// steps at 256 x 64 with 32, 16, 8, 4 rows (216, 408, 792, 1584 waves): 2800, 2647,
+// 2570, 2567 us; one of 1024 x 256 (3168 waves with 32): 782, 779, 793, 844 us.
+int xs_rows(int nx, int ny) {
+  int rows = 32;
+  while (rows > 8 && 2 * NU * ((ny + 63) / 64) * xs_segments(nx, rows) < 1024) rows /= 2;
+  return rows;
+}
+
+// Flux VJP of one RK stage with input (Us, As), whose primitives are in w.qb, and
+// rhs cotangent rb; the results are added into (Ut, At).
 void flux_vjp(jh_ctx* c, const AdjArgs& a, AdjWork& w, const double* Us, const double* As,
               const double* rb, const unsigned long long* alpha, double* Ut, double* At) {
   hipStream_t st = c->stream;
-  const int n = a.nx * a.ny;
-  adj_prim_kernel<<<blocks_for(n), 256, 0, st>>>(a, Us, As, w.qb);
-  flux_vjp_x_kernel<<<xs_blocks(a.nx, a.ny), 256, 0, st>>>(a, Us, w.qb, rb, alpha, w.hx);
+  const int xseg = xs_rows(a.nx, a.ny);
+  flux_vjp_x_kernel<<<xs_blocks(a.nx, a.ny, xseg), 256, 0, st>>>(a, Us, w.qb, rb, alpha, w.hx,
+                                                                 xseg);
   flux_vjp_y_kernel<<<w.nblk, 64 * kYRows, 0, st>>>(a, Us, As, rb, alpha, w.hx, Ut, At, w.Ubp,
                                                     w.abp, w.spd, w.part);
   alpha_reduce_kernel<<<1, 256, 0, st>>>(w.part, w.nblk, w.scal, w.amx, w.cnt);
@@ -719,15 +729,15 @@ int vjp_reverse(jh_ctx* c, AdjWork& w, double dt, const unsigned long long* cons
   // reverse of the stage's combine
   // stage 3: U3 = 1/3 U + 2/3 (U2 + r(U2))
   getT_split_kernel<<<bc1, 256, 0, st>>>(aa, w.U[3], w.A[3], 1.0 / 3.0, 0.0, 2.0 / 3.0, w.Ub,
-                                         w.Uacc, w.rb, w.ab);
+                                         w.Uacc, w.rb, w.ab, w.U[2], w.A[2], w.qb);
   flux_vjp(c, aa, w, w.U[2], w.A[2], w.rb, alpha[2], w.Ub, w.ab);
   // stage 2: U2 = 3/4 U + 1/4 (U1 + r(U1))
   getT_split_kernel<<<bc1, 256, 0, st>>>(aa, w.U[2], w.A[2], 3.0 / 4.0, 1.0, 1.0 / 4.0, w.Ub,
-                                         w.Uacc, w.rb, w.ab);
+                                         w.Uacc, w.rb, w.ab, w.U[1], w.A[1], w.qb);
   flux_vjp(c, aa, w, w.U[1], w.A[1], w.rb, alpha[1], w.Ub, w.ab);
   // stage 1: U1 = U + r(U)
   getT_split_kernel<<<bc1, 256, 0, st>>>(aa, w.U[1], w.A[1], 1.0, 1.0, 0.0, w.Ub, w.Uacc,
-                                         nullptr, w.ab);
+                                         nullptr, w.ab, w.U[0], w.A[0], w.qb);
   flux_vjp(c, aa, w, w.U[0], w.A[0], w.Ub, alpha[0], w.Uacc, w.ab);
   return check_launch(c, "vjp kernels");
 }

@@ -178,25 +178,28 @@ namespace jh {
 
 // Reverse of get_T_nasa7 at the converged T (get_T_bwd,
 // thermo_model.py:159-188): (gamma_bar, T_bar) -> (e_bar, Y_bar[0:NS-1]).
-// Y is the filled mass-fraction vector, R its gas constant.
-__host__ __device__ __forceinline__ void getT_vjp(const MechConst& c, const double (&Y)[JH_NS],
-                                                  double R, double T, double gb, double Tbr,
-                                                  double& eb, double (&Yb)[JH_NS - 1]) {
-  const int r = T < c.Tcr ? 0 : 1;
+// Y is the filled mass-fraction vector, R its gas constant; tab the mixture tables
+// (c, or their copy in LDS: the range index is per lane).
+template <typename Tab>
+__host__ __device__ __forceinline__ void getT_vjp(const MechConst& c, const Tab& tab,
+                                                  const double (&Y)[JH_NS], double R, double T,
+                                                  double gb, double Tbr, double& eb,
+                                                  double (&Yb)[JH_NS - 1]) {
+  const int r = T < tab.Tcr ? 0 : 1;
   double cpk[JH_NS], ek[JH_NS];
   double cp = 0.0, dcp = 0.0;
 #pragma unroll
   for (int k = 0; k < JH_NS; ++k) {
-    double a = c.cp[r][k][0];
+    double a = tab.cp[r][k][0];
 #pragma unroll
-    for (int j = 1; j < 5; ++j) a = a * T + c.cp[r][k][j];
-    double d = 4.0 * c.cp[r][k][0];
-    d = d * T + 3.0 * c.cp[r][k][1];
-    d = d * T + 2.0 * c.cp[r][k][2];
-    d = d * T + c.cp[r][k][3];
-    double h = c.h[r][k][0];
+    for (int j = 1; j < 5; ++j) a = a * T + tab.cp[r][k][j];
+    double d = 4.0 * tab.cp[r][k][0];
+    d = d * T + 3.0 * tab.cp[r][k][1];
+    d = d * T + 2.0 * tab.cp[r][k][2];
+    d = d * T + tab.cp[r][k][3];
+    double h = tab.h[r][k][0];
 #pragma unroll
-    for (int j = 1; j < 6; ++j) h = h * T + c.h[r][k][j];
+    for (int j = 1; j < 6; ++j) h = h * T + tab.h[r][k][j];
     cpk[k] = a;
     ek[k] = h - c.R[k] * T;
     cp += a * Y[k];
@@ -216,6 +219,12 @@ __host__ __device__ __forceinline__ void getT_vjp(const MechConst& c, const doub
     const double dgdY = dgdT * dTdY + (dcpdY * cv - dcvdY * cp) * icv * icv;
     Yb[k] = gb * dgdY + Tbr * dTdY;
   }
+}
+
+__host__ __device__ __forceinline__ void getT_vjp(const MechConst& c, const double (&Y)[JH_NS],
+                                                  double R, double T, double gb, double Tbr,
+                                                  double& eb, double (&Yb)[JH_NS - 1]) {
+  getT_vjp(c, c, Y, R, T, gb, Tbr, eb, Yb);
 }
 
 }  // namespace jh
