@@ -92,48 +92,6 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
   constexpr double sc = LfScale<W>::value;   // split fluxes scaled as stage_body's
   constexpr W hs = (W)(0.5 * sc);
   const double idx = 1.0 / sc / a.dx, idy = 1.0 / sc / a.dy;
-  double alx, aly;
-  if constexpr (ADDR == ADDR_LEVEL) {
-    // the block's LF maxima: its interior cells' (reduced by the producer) and
-    // its ghost cells', which are copies of interior cells with the momenta
-    // negated at most, through the index table
-    const int PY = ny + 6, P = (nx + 6) * PY, ring = P - nx * ny;
-    double mx = 0.0, my = 0.0;
-    for (int r = t; r < ring; r += blockDim.x) {
-      int p;
-      if (r < 6 * PY) {                    // rows 0-2 and nx+3..nx+5 whole
-        p = r < 3 * PY ? r : r + nx * PY;
-      } else {                             // the 6 ghost columns of the rows between
-        const int k = r - 6 * PY, row = k / 6, col = k - row * 6;
-        p = (3 + row) * PY + (col < 3 ? col : ny + col);
-      }
-      const int s = lv->idx[(size_t)blk * P + p];
-      mx = fmax(mx, lv->spd[s]);
-      my = fmax(my, lv->spd[lv->ncell + s]);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      mx = fmax(mx, __shfl_xor(mx, off, 64));
-      my = fmax(my, __shfl_xor(my, off, 64));
-    }
-    const int nw = blockDim.x >> 6;
-    if ((t & 63) == 0) {
-      red[w] = mx;
-      red[16 + w] = my;
-    }
-    __syncthreads();
-    alx = fmax(bitsd(a.sc->amax[0][stage][0]), red[0]);
-    aly = fmax(bitsd(a.sc->amax[0][stage][1]), red[16]);
-    for (int i = 1; i < nw; ++i) {
-      alx = fmax(alx, red[i]);
-      aly = fmax(aly, red[16 + i]);
-    }
-  } else {
-    alx = bitsd(a.sc->amax[a.parity][stage][0]);
-    aly = bitsd(a.sc->amax[a.parity][stage][1]);
-  }
-  const W hax = hs * (W)(Real)alx, hay = hs * (W)(Real)aly;
-
   // ---- the thread's cells: slot 0 = interior cell tg, then halo cells ----
   constexpr int NS = 1 + NH;
   const int ncell = ct.cells(), nhalo = ct.halo();
@@ -246,6 +204,49 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
     if ((flips >> (2 * s)) & 1u) q[s].u = -q[s].u;
     if ((flips >> (2 * s)) & 2u) q[s].v = -q[s].v;
   }
+  double alx, aly;
+  if constexpr (ADDR == ADDR_LEVEL) {
+    // the block's LF maxima: its interior cells' (reduced by the producer) and
+    // its ghost cells', which are copies of interior cells with the momenta
+    // negated at most, through the index table; after the state's reads, which
+    // cover the table's (mixed level of 1000 blocks: 958 -> 945 us a step)
+    const int PY = ny + 6, P = (nx + 6) * PY, ring = P - nx * ny;
+    double mx = 0.0, my = 0.0;
+    for (int r = t; r < ring; r += blockDim.x) {
+      int p;
+      if (r < 6 * PY) {                    // rows 0-2 and nx+3..nx+5 whole
+        p = r < 3 * PY ? r : r + nx * PY;
+      } else {                             // the 6 ghost columns of the rows between
+        const int k = r - 6 * PY, row = k / 6, col = k - row * 6;
+        p = (3 + row) * PY + (col < 3 ? col : ny + col);
+      }
+      const int s = lv->idx[(size_t)blk * P + p];
+      mx = fmax(mx, lv->spd[s]);
+      my = fmax(my, lv->spd[lv->ncell + s]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      mx = fmax(mx, __shfl_xor(mx, off, 64));
+      my = fmax(my, __shfl_xor(my, off, 64));
+    }
+    const int nw = blockDim.x >> 6;
+    if ((t & 63) == 0) {
+      red[w] = mx;
+      red[16 + w] = my;
+    }
+    __syncthreads();
+    alx = fmax(bitsd(a.sc->amax[0][stage][0]), red[0]);
+    aly = fmax(bitsd(a.sc->amax[0][stage][1]), red[16]);
+    for (int i = 1; i < nw; ++i) {
+      alx = fmax(alx, red[i]);
+      aly = fmax(aly, red[16 + i]);
+    }
+  } else {
+    alx = bitsd(a.sc->amax[a.parity][stage][0]);
+    aly = bitsd(a.sc->amax[a.parity][stage][1]);
+  }
+  const W hax = hs * (W)(Real)alx, hay = hs * (W)(Real)aly;
+
   const int gx = x0 + xr, gy = y0 + yc;
   const bool own = has[0] && gx < nx && gy < ny;
   const int n = ADDR == ADDR_PAD ? (nx + 6) * (ny + 6) : nx * ny;
