@@ -39,6 +39,15 @@ __host__ __device__ __forceinline__ void gibbs(const Tab& c, double T, double in
   }
 }
 
+// Whether v holds in any lane of the wave.
+__host__ __device__ __forceinline__ bool any_lane(bool v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __any(v);
+#else
+  return v;
+#endif
+}
+
 // Solve A x = b in place (b <- x) by LU with partial pivoting, the
 // factorisation jnp.linalg.solve uses (LAPACK getrf/getrs).  Row swaps are
 // predicated selects so every index stays compile-time and A lives in VGPRs.
@@ -49,26 +58,26 @@ __host__ __device__ __forceinline__ bool lu_solve(double (&A)[N][N], double (&b)
   bool ok = true;
 #pragma unroll
   for (int col = 0; col < N; ++col) {
-    int p = col;
     double amax = fabs(A[col][col]);
+    // the search for the pivot and the predicated swap only where a lane of the
+    // wave pivots in this column, and there only of the rows some lane takes
+    bool swaps = false;
 #pragma unroll
-    for (int r = col + 1; r < N; ++r) {
-      const double v = fabs(A[r][col]);
-      if (v > amax) {
-        amax = v;
-        p = r;
+    for (int r = col + 1; r < N; ++r) swaps = swaps || fabs(A[r][col]) > amax;
+    if (any_lane(swaps)) {
+      int p = col;
+#pragma unroll
+      for (int r = col + 1; r < N; ++r) {
+        const double v = fabs(A[r][col]);
+        if (v > amax) {
+          amax = v;
+          p = r;
+        }
       }
-    }
-    // the predicated swap is skipped when no lane of the wave pivots
-#if defined(__HIP_DEVICE_COMPILE__)
-    const bool any_swap = __any(p != col);
-#else
-    const bool any_swap = p != col;
-#endif
-    if (any_swap) {
 #pragma unroll
       for (int r = col + 1; r < N; ++r) {
         const bool s = (p == r);
+        if (!any_lane(s)) continue;
 #pragma unroll
         for (int j = col; j < N; ++j) {
           const double t = A[col][j];
