@@ -155,6 +155,23 @@ __device__ __forceinline__ void godunov_stage_body(const StepArgs<Real>& a, int 
     }
   }
   hllc_flux<Real, 1>(c, L.mix, qL, qR, Fl);
+  // the own cell (x0 + w, y0 + ly) and its U^n, all planes at once and ahead of the
+  // stores: U^n may be the output's memory, so a plane read after a store would wait
+  // for it (FP64 stage of 1500 x 300 cells: 122 -> 118 us)
+  const int gx = x0 + w, gy = y0 + ly;
+  const bool own = w < TX && gx < nx && gy < ny;
+  const int o = own ? gx * ny + gy : 0;
+  Real uc[NU], u0[NU];
+  Real T0 = (Real)0;
+  if (MODE != MODE_RHS) {
+#pragma unroll
+    for (int cv = 0; cv < NU; ++cv) uc[cv] = (Us + (size_t)cv * n)[o];
+    if (stage != 0) {
+#pragma unroll
+      for (int cv = 0; cv < NU; ++cv) u0[cv] = (Un + (size_t)cv * n)[o];
+    }
+    T0 = (auxs + n)[o];
+  }
   if (w == TX && ly < TX) {
 #pragma unroll
     for (int cv = 0; cv < NU; ++cv) L.Ge[cv][ly] = Fl[cv];
@@ -162,10 +179,7 @@ __device__ __forceinline__ void godunov_stage_body(const StepArgs<Real>& a, int 
   __syncthreads();
   if (w >= TX) return;
 
-  // ---------------- divergence + RK combine for cell (x0 + w, y0 + ly)
-  const int gx = x0 + w, gy = y0 + ly;
-  const bool own = gx < nx && gy < ny;
-  const int o = gx * ny + gy;
+  // ---------------- divergence + RK combine
   const double dt = step_dt(a);
   const double idx = 1.0 / a.dx, idy = 1.0 / a.dy;
   double un[NU];       // FP64 whatever Real (see stage_body)
@@ -179,14 +193,10 @@ __device__ __forceinline__ void godunov_stage_body(const StepArgs<Real>& a, int 
     if (MODE == MODE_RHS) {
       un[cv] = rhs;
     } else {
-      const double uc = own ? (double)Us[cv * n + o] : 0.0;
-      if (stage == 0) {
-        un[cv] = uc + rhs;
-      } else {
-        const double u0 = own ? (double)Un[cv * n + o] : 0.0;
-        if (stage == 1) un[cv] = (3.0 / 4.0) * u0 + (1.0 / 4.0) * (uc + rhs);
-        else un[cv] = (1.0 / 3.0) * u0 + (2.0 / 3.0) * (uc + rhs);
-      }
+      const double c0 = (double)uc[cv];
+      if (stage == 0) un[cv] = c0 + rhs;
+      else if (stage == 1) un[cv] = (3.0 / 4.0) * (double)u0[cv] + (1.0 / 4.0) * (c0 + rhs);
+      else un[cv] = (1.0 / 3.0) * (double)u0[cv] + (2.0 / 3.0) * (c0 + rhs);
     }
     if (own) Uo[cv * n + o] = (Real)un[cv];
   }
@@ -207,7 +217,7 @@ __device__ __forceinline__ void godunov_stage_body(const StepArgs<Real>& a, int 
 #pragma unroll
     for (int k = 0; k < JH_NS - 1; ++k) Y[k] = us[4 + k] * ir;
     const double R = fill_Y_get_R(c, Y);
-    double T = (double)auxs[n + o];
+    double T = (double)T0;
     double gamma;
     bool conv;
     if (a.hside) {
