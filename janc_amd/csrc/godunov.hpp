@@ -113,10 +113,8 @@ __device__ __forceinline__ void godunov_stage_body(const StepArgs<Real>& a, int 
       for (int h = 0; h < NSX; ++h) gcell_advance(cell[h], cv);
       __syncthreads();
       const int col = ly + 3;
-      qL[cv] = recon_L<RECON, Real>(Q[w][col], Q[w + 1][col], Q[w + 2][col], Q[w + 3][col],
-                                    Q[w + 4][col]);
-      qR[cv] = recon_R<RECON, Real>(Q[w + 1][col], Q[w + 2][col], Q[w + 3][col],
-                                    Q[w + 4][col], Q[w + 5][col]);
+      recon_LR<RECON, Real>(Q[w][col], Q[w + 1][col], Q[w + 2][col], Q[w + 3][col],
+                            Q[w + 4][col], Q[w + 5][col], qL[cv], qR[cv]);
     }
   }
   hllc_flux<Real, 0>(c, L.mix, qL, qR, Fl);
@@ -148,10 +146,8 @@ __device__ __forceinline__ void godunov_stage_body(const StepArgs<Real>& a, int 
       if (has) Q[qr][qc] = gcell_q(cell, cv);
       gcell_advance(cell, cv);
       __syncthreads();
-      qL[cv] = recon_L<RECON, Real>(Q[fr][fc], Q[fr][fc + 1], Q[fr][fc + 2], Q[fr][fc + 3],
-                                    Q[fr][fc + 4]);
-      qR[cv] = recon_R<RECON, Real>(Q[fr][fc + 1], Q[fr][fc + 2], Q[fr][fc + 3],
-                                    Q[fr][fc + 4], Q[fr][fc + 5]);
+      recon_LR<RECON, Real>(Q[fr][fc], Q[fr][fc + 1], Q[fr][fc + 2], Q[fr][fc + 3],
+                            Q[fr][fc + 4], Q[fr][fc + 5], qL[cv], qR[cv]);
     }
   }
   hllc_flux<Real, 1>(c, L.mix, qL, qR, Fl);

