@@ -37,6 +37,7 @@ struct jh_ctx {
   int parity = 0;
   bool user_filled[4] = {false, false, false, false};   // JH_BC_USER strips written
   int tile = 0;                   // stage-kernel variant (kTileRows / kTileWaves)
+  bool tile_chosen = false;       // by jh_ctx_set_tile
   CompactTile compact{0, 0, 0, 0};   // small grids: the compact kernel's tile (R = 0: none)
   int solver = JH_SOLVER_FLUX_SPLITTING;   // jh_ctx_set_flux
   int split = JH_SPLIT_LF;
@@ -224,6 +225,19 @@ constexpr int kTileVariants = 5;
 constexpr int kTileRows[kTileVariants] = {8, 8, 16, 16, 32};
 constexpr int kTileWaves[kTileVariants] = {3, 4, 4, 5, 4};
 
+// Default variant, by the number of 16-row tiles: FP64 takes 16 rows (two blocks of
+// eight waves fill a CU's LDS; 8 rows at 4000 x 500: 2085 us for two steps, 16: 2045).
+// Mixed takes 16 rows while their tiles are at most two rounds of the chip, for their
+// smaller halo, and 8 rows beyond, whose blocks of four waves wait less at their
+// barriers: microseconds a step with 16 / 8 rows at 256 tiles 158 / 162, 470 tiles 225 /
+// 231, 1000 tiles 401 / 401, 1750 tiles 733 / 712, 3008 tiles 1182 / 1158, 4000 tiles
+// 1526 / 1485, 64 uneven cases of 6868 tiles 2679 / 2554.
+// MUSCL's lighter faces keep 16 rows (1750 tiles 613 / 620, 3008 tiles 1011 / 1024).
+int default_tile(int precision, long long tiles16, int recon = JH_RECON_WENO5_JS) {
+  if (precision == JH_PREC_FP64) return 3;
+  return tiles16 <= 1024 || recon != JH_RECON_WENO5_JS ? 2 : 1;
+}
+
 // With the grid-wide temperature-solve stop the flux-splitting stage kernel
 // runs one tile shape (its epilogue carries the per-candidate maxima): 16
 // rows at a 4-wave register budget, whatever the context's variant.
@@ -346,6 +360,11 @@ void launch_stage(jh_ctx* c, const StepArgs<Real>& a, int stage, const Real* Us,
   } else {
     launch_split_stage<Real, MODE, RECON_WENO5>(c, a, stage, Us, As, Un, Uo, Ao);
   }
+}
+
+int ctx_default_tile(const jh_ctx* c) {
+  return default_tile(c->precision, (long long)((c->nx + 15) / 16) * ((c->ny + TY - 1) / TY),
+                      c->recon);
 }
 
 int tile_rows(const jh_ctx* c) { return kTileRows[c->tile]; }
@@ -1215,10 +1234,7 @@ int jh_ctx_create(int nx, int ny, double dx, double dy, const int* bc_kind,
   c->dx = dx;
   c->dy = dy;
   c->precision = precision;
-  // default stage-kernel variant (the autotuner's usual pick on MI355X):
-  // 16 rows with the 5-wave register budget for FP64, 16 rows at 4 waves/SIMD
-  // for the mixed form
-  c->tile = precision == JH_PREC_FP64 ? 3 : 2;
+  c->tile = ctx_default_tile(c);
   const int rule = compact_rule(c);
   if (rule >= 0)
     c->compact = compact_tile(nx, ny, kCompactRules[rule].threads, kCompactRules[rule].halo);
@@ -1297,6 +1313,7 @@ int jh_ctx_set_tile(jh_ctx* c, int variant) {
   if (!c) return JH_ERR_ARG;
   if (variant < 0 || variant >= jh_tile_variants()) return fail(c, JH_ERR_ARG, "unknown tile variant");
   c->tile = variant;
+  c->tile_chosen = true;
   return JH_OK;
 }
 
@@ -1359,6 +1376,7 @@ int jh_ctx_set_flux(jh_ctx* c, int solver_type, int split_method, int reconstruc
   c->solver = solver_type;
   c->split = split_method;
   c->recon = reconstruction;
+  if (!c->tile_chosen) c->tile = ctx_default_tile(c);
   return JH_OK;
 }
 
@@ -1691,7 +1709,6 @@ int jh_batch_create(int ncase, const int* nx, const int* ny, const double* dx, c
   jh_batch* b = new jh_batch();
   b->ncase = ncase;
   b->precision = precision;
-  b->tile = precision == JH_PREC_FP64 ? 3 : 2;   // as jh_ctx_create
   b->user = static_cast<hipStream_t>(stream);
   b->nx.assign(nx, nx + ncase);
   b->ny.assign(ny, ny + ncase);
@@ -1729,6 +1746,7 @@ int jh_batch_create(int ncase, const int* nx, const int* ny, const double* dx, c
     b->h_off[b->t_red + k + 1] = b->h_off[b->t_red + k] + std::min(cb, 64);
     b->h_off[b->t_chem + k + 1] = b->h_off[b->t_chem + k] + cb;
   }
+  b->tile = default_tile(precision, b->h_off[b->t_stage[2] + ncase]);
   const size_t es = precision == JH_PREC_FP64 ? 8 : 4;
   size_t total = 0;
   b->buf_off.resize(ncase);
