@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void level_speeds_kernel(StepArgs<Real> a, lon
   for (int l = threadIdx.x; l < n; l += blockDim.x) {
     const int x = l / a.ny, i = b * n + l;
     const Real* p = U + b * sb + x * sr + (l - x * a.ny);
-    const Prim<double> q = cell_prim<double, true>(*a.mc, p, p + NU * splane, (int)splane);
+    const Prim<double> q = cell_prim<double, true>(*a.mc, p, p + NU * splane, splane);
     const double sx = nan_to_zero(fabs(q.u) + q.a), sy = nan_to_zero(fabs(q.v) + q.a);
     spd[i] = sx;
     spd[ncell + i] = sy;

@@ -114,7 +114,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
     else if constexpr (ADDR == ADDR_STRIP) return locate<Real>(a, Us, auxs, gx, gy);
     else {
       CellRef<Real> r;
-      r.stride = (int)lv->splane;
+      r.stride = 0;                    // planes are lv->splane apart (plane)
       const bool inx = gx >= 0 && gx < nx, iny = gy >= 0 && gy < ny;
       r.ok = gx >= -3 && gx < nx + 3 && gy >= -3 && gy < ny + 3;
       long long o = 0;
@@ -130,6 +130,12 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
       r.x = r.u + NU * lv->splane;
       return r;
     }
+  };
+  // Element v planes from a cell.  The planes of a level's interiors are the
+  // caller's view: their stride may be of any size.
+  const auto plane = [&](const CellRef<Real>& r, int v) -> Real {
+    if constexpr (ADDR == ADDR_LEVEL) return r.u[v * lv->splane];
+    else return r.u[(size_t)v * r.stride];
   };
   CellRef<Real> ref[NS];
   Prim<W> q[NS];
@@ -162,7 +168,11 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
   if constexpr (G == 1) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      if (ref[s].ok) q[s] = cell_prim<W, false, Real>(c, ref[s].u, ref[s].x, ref[s].stride);
+      if (!ref[s].ok) continue;
+      if constexpr (ADDR == ADDR_LEVEL)
+        q[s] = cell_prim<W, false>(c, ref[s].u, ref[s].x, lv->splane);
+      else
+        q[s] = cell_prim<W, false>(c, ref[s].u, ref[s].x, ref[s].stride);
     }
   } else {
     // the region's primitives once per block, through LDS
@@ -179,7 +189,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
       unsigned int f;
       const CellRef<Real> r = find(x0 + lx, y0 + ly, f);
       if (r.ok) {
-        const Prim<W> p = cell_prim<W, false, Real>(c, r.u, r.x, r.stride);
+        const Prim<W> p = cell_prim<W, false>(c, r.u, r.x, r.stride);
         sP[i] = p.rho;
         sP[nreg + i] = p.u;
         sP[2 * nreg + i] = p.v;
@@ -305,7 +315,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
   const int cv0 = g * NVG;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
-    nxt[s] = ref[s].ok ? ref[s].u[(size_t)cv0 * ref[s].stride] : (Real)0;
+    nxt[s] = ref[s].ok ? plane(ref[s], cv0) : (Real)0;
 #pragma unroll 1
   for (int k = 0; k < NVG; ++k) {
     const int cv = cv0 + k;
@@ -323,7 +333,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
     if (k + 1 < NVG) {
 #pragma unroll
       for (int s = 0; s < NS; ++s)
-        if (ref[s].ok) nxt[s] = ref[s].u[(size_t)(cv + 1) * ref[s].stride];
+        if (ref[s].ok) nxt[s] = plane(ref[s], cv + 1);
     }
     W u0n = (W)0;
     if (MODE != MODE_RHS && stage != 0 && own) u0n = (W)Un[unidx + cv * unstride];
@@ -375,7 +385,7 @@ __device__ __forceinline__ void compact_body(const StepArgs<Real>& a, const Comp
 #pragma unroll
     for (int k = 0; k < JH_NS - 1; ++k) Y[k] = (double)un[(4 + k) * st] * ir;
     const double Rg = fill_Y_get_R(c, Y);
-    double T = (double)ref[0].x[ref[0].stride];
+    double T = (double)(ADDR == ADDR_LEVEL ? plane(ref[0], NU + 1) : ref[0].x[ref[0].stride]);
     double gamma;
     const bool conv = halley_T(mix, Y, Rg, e, T, gamma);
     auxo[oidx] = (Real)gamma;

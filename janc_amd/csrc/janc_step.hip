@@ -2058,8 +2058,7 @@ int jh_blocks_level_step(jh_blocks* b, int n_blk, const void* blk, long long sb,
   if (!blk || !idx || !s_u || !s_v || !work || !out) return kfail(b, JH_ERR_ARG, "NULL pointer");
   if (out == blk) return kfail(b, JH_ERR_ARG, "out must not alias the blocks");
   if (!(dt > 0)) return kfail(b, JH_ERR_ARG, "dt must be > 0");
-  if (sb < 1 || sv < 1 || sr < b->ny || sv >= (1ll << 31))
-    return kfail(b, JH_ERR_ARG, "bad strides");
+  if (sb < 1 || sv < 1 || sr < b->ny) return kfail(b, JH_ERR_ARG, "bad strides");
   int rc = blocks_checks(b, n_blk);
   if (rc) return rc;
   if (b->precision == JH_PREC_FP64)

@@ -275,9 +275,11 @@ __device__ __forceinline__ Prim<W> cell_prim_ld(const MechConst& c, const Load& 
   return q;
 }
 
-template <typename W, bool WITH_A, typename Real>
+// stride: int where 13 planes of the state stay below 2^31 elements (the
+// contexts' and padded blocks' own planes), wider for a caller's strided view.
+template <typename W, bool WITH_A, typename Real, typename Stride>
 __device__ __forceinline__ Prim<W> cell_prim(const MechConst& c, const Real* __restrict__ Up,
-                                             const Real* __restrict__ ap, int stride) {
+                                             const Real* __restrict__ ap, Stride stride) {
   return cell_prim_ld<W, WITH_A>(c, [&](int v) { return v < 12 ? Up[v * stride]
                                                                : ap[(v - 12) * stride]; });
 }

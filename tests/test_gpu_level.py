@@ -1,0 +1,40 @@
+"""The step of a uniform block level on its own grid (blocks read in place)
+against the padded path, bit for bit."""
+import pytest
+
+from janc_amd import cases
+from janc_amd.mechanism import Mechanism
+
+torch = pytest.importorskip("torch")
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+
+DTYPE = {"fp64": torch.float64, "mixed": torch.float32}
+
+
+@pytest.mark.parametrize("precision,stride", [("mixed", 195225787), ("fp64", 195225787),
+                                              ("mixed", 2 ** 31 + 6)])
+def test_plane_stride_of_any_size(precision, stride):
+    """A level that is a view into a plane-major buffer: 11 planes are 2^31
+    elements apart from the first stride on, one plane from the last."""
+    from janc_amd.amr import BlockSolver, UniformBlockGrid
+    U, aux, g = cases.detonation_tube(Mechanism(), nx=12, ny=14, driver=3)
+    sol = BlockSolver(cases.simulation_config(g, dt=1e-9, precision=precision))
+    grid = UniformBlockGrid(g["boundary_config"], 2, 2, 6, 7)
+    blk = grid.split(torch.as_tensor(U).to(dtype=DTYPE[precision]).cuda(),
+                     torch.as_tensor(aux).to(dtype=DTYPE[precision]).cuda())
+    count = 13 * stride + 4 * 42
+    if torch.cuda.mem_get_info()[0] < count * blk.element_size() + 2 ** 31:
+        pytest.skip("needs %d GB" % (count * blk.element_size() >> 30))
+    buf = torch.empty((count,), dtype=blk.dtype, device="cuda")
+    far = buf.as_strided(tuple(blk.shape), (42, stride, 7, 1))
+    for v in range(14):
+        far[:, v].copy_(blk[:, v])
+    torch.cuda.synchronize()
+    print("level in place", precision, stride, flush=True)
+    args = (1, None, g["dx"], g["dy"], 1e-9)
+    got = sol.advance_one_step(*args, far, None, amr=grid)
+    ref = sol.advance_one_step(*args, blk, None, amr=grid)
+    assert torch.isfinite(ref).all() and torch.equal(got, ref)
+    del far, buf
+    torch.cuda.empty_cache()
