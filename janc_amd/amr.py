@@ -135,7 +135,7 @@ class BlockSolver:
         if amr is None:
             raise ValueError("advance_one_step needs the AMR hierarchy's ghost functions "
                              "(jaxamr's amr module or an object with the same two functions)")
-        if type(amr) is UniformBlockGrid and ref_blk_data.is_cuda:
+        if type(amr) is UniformBlockGrid and amr.own_ghosts() and ref_blk_data.is_cuda:
             return self._level_step(amr, ref_blk_data, dx, dy, dt)
         g0 = amr.get_ghost_block_data(ref_blk_data, ref_blk_info)
         b = None
@@ -294,6 +294,12 @@ class UniformBlockGrid:
         full = b.permute(2, 0, 3, 1, 4).reshape(nv, self.nbx * self.bnx, self.nby * self.bny)
         return full[:-2], full[-2:]
 
+    def own_ghosts(self):
+        """Whether the two ghost functions are the class's own: a caller may
+        replace them (on the object or the class), and is asked then."""
+        return tuple(getattr(f, "__func__", None) for f in
+                     (self.get_ghost_block_data, self.update_external_boundary)) == _GHOSTS
+
     def gpu_tables(self, blk):
         """Momentum signs in blk's type, after checking that blk is this
         level's interiors on the grid's device."""
@@ -339,3 +345,6 @@ class UniformBlockGrid:
         """A single level: the interiors are the blocks (on the GPU the view
         itself; get_ghost_block_data reads it through its strides)."""
         return interiors if interiors.is_cuda else interiors.contiguous()
+
+
+_GHOSTS = (UniformBlockGrid.get_ghost_block_data, UniformBlockGrid.update_external_boundary)

@@ -38,3 +38,31 @@ def test_plane_stride_of_any_size(precision, stride):
     assert torch.isfinite(ref).all() and torch.equal(got, ref)
     del far, buf
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("name,where", [("get_ghost_block_data", "object"),
+                                        ("update_external_boundary", "object"),
+                                        ("get_ghost_block_data", "class"),
+                                        ("update_external_boundary", "class")])
+def test_replaced_ghost_functions_are_asked(name, where, monkeypatch):
+    """A caller's own ghost function, put on a UniformBlockGrid or on the
+    class, is called for every stage and its result used."""
+    from janc_amd.amr import BlockSolver, UniformBlockGrid
+    U, aux, g = cases.detonation_tube(Mechanism(), nx=12, ny=14, driver=3)
+    sol = BlockSolver(cases.simulation_config(g, dt=1e-9))
+    grid = UniformBlockGrid(g["boundary_config"], 2, 2, 6, 7)
+    blk = grid.split(torch.as_tensor(U).cuda(), torch.as_tensor(aux).cuda())
+    own, calls = getattr(grid, name), []
+
+    def replaced(*args):
+        calls.append(name)
+        out = own(*args[1:] if where == "class" else args).clone()
+        out[:, 2] += 1.0                       # the caller's change of rho v
+        return out
+
+    args = (1, None, g["dx"], g["dy"], 1e-9, blk, None)
+    plain = sol.advance_one_step(*args, amr=grid)
+    monkeypatch.setattr(grid if where == "object" else UniformBlockGrid, name, replaced)
+    out = sol.advance_one_step(*args, amr=grid)
+    assert calls == [name] * 3
+    assert not torch.equal(out, plain)
