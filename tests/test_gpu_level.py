@@ -66,3 +66,45 @@ def test_replaced_ghost_functions_are_asked(name, where, monkeypatch):
     out = sol.advance_one_step(*args, amr=grid)
     assert calls == [name] * 3
     assert not torch.equal(out, plain)
+
+
+# left, right, bottom, top: both momenta flipped on one ghost, copies across the
+# domain with the off-by-one pre-pad, each alone and against a wall
+KINDS = [("no_slip_wall", "no_slip_wall", "no_slip_wall", "no_slip_wall"),
+         ("periodic", "periodic", "periodic", "periodic"),
+         ("periodic", "periodic", "no_slip_wall", "slip_wall"),
+         ("slip_wall", "no_slip_wall", "periodic", "periodic"),
+         ("slip_wall", "slip_wall", "slip_wall", "zero_gradient")]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kinds", KINDS)
+def test_boundary_kinds(kinds, precision):
+    """Every copied ghost kind, with momenta at the edges that a wrong or
+    missing flip or source cell would show in; the two steps of the level read
+    in place equal the padded path's."""
+    from janc_amd.amr import BlockSolver, UniformBlockGrid
+
+    class Padded(UniformBlockGrid):
+        pass
+
+    nbx, nby, bnx, bny = 3, 2, 11, 19
+    U, aux, g = cases.detonation_tube(Mechanism(), nx=nbx * bnx, ny=nby * bny, driver=8)
+    gen = torch.Generator().manual_seed(5)
+    U, aux = torch.as_tensor(U).clone(), torch.as_tensor(aux)
+    noise = 200.0 * (torch.rand((2,) + tuple(U.shape[1:]), generator=gen,
+                                dtype=torch.float64) - 0.4)
+    kin = 0.5 * (U[1] ** 2 + U[2] ** 2) / U[0]
+    U[1:3] += U[0] * noise
+    U[3] += 0.5 * (U[1] ** 2 + U[2] ** 2) / U[0] - kin
+    bc = dict(zip(("left_boundary", "right_boundary", "bottom_boundary", "top_boundary"), kinds))
+    sol = BlockSolver(cases.simulation_config(dict(g, boundary_config=bc), dt=2e-9,
+                                              precision=precision))
+    out = []
+    for cls in (UniformBlockGrid, Padded):
+        grid = cls(bc, nbx, nby, bnx, bny)
+        blk = grid.split(U.to(DTYPE[precision]).cuda(), aux.to(DTYPE[precision]).cuda())
+        for _ in range(2):
+            blk = sol.advance_one_step(1, None, g["dx"], g["dy"], 2e-9, blk, None, amr=grid)
+        out.append(blk)
+    assert torch.isfinite(out[0]).all() and torch.equal(out[0], out[1])
