@@ -111,9 +111,12 @@ int jh_ctx_set_flux(jh_ctx* ctx, int solver_type, int split_method, int reconstr
  * shape per reconstruction (WENO5_JS: 64 x 3 cells, 256 threads; MUSCL:
  * 64 x 7 cells, 512 threads), the Steger-Warming kernel one (64 x 16 cells,
  * 512 threads).  Grids of up to 200000 cells run a kernel of smaller tiles
- * under LF splitting with WENO5_JS, whatever the variant. */
+ * under LF splitting with WENO5_JS, whatever the variant.
+ * jh_ctx_compact: 1 if the context's RK stages run the kernel of smaller
+ * tiles, 0 if not. */
 int jh_ctx_set_tile(jh_ctx* ctx, int variant);
 int jh_ctx_get_tile(const jh_ctx* ctx);
+int jh_ctx_compact(const jh_ctx* ctx);
 
 /* Stop rule of the Halley temperature solve after every RK stage, after the
  * chemistry and in jh_update_aux (get_T_nasa7, model/thermo_model.py:

@@ -45,6 +45,7 @@ SIGNATURES = {
     "jh_ctx_set_stream": (_c_int, [_vp, _vp]),
     "jh_ctx_set_inlet": (_c_int, [_vp, _c_double, ctypes.POINTER(_c_double), _c_int]),
     "jh_ctx_set_tile": (_c_int, [_vp, _c_int]),
+    "jh_ctx_compact": (_c_int, [_vp]),
     "jh_ctx_set_flux": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int]),
     "jh_ctx_get_tile": (_c_int, [_vp]),
     "jh_ctx_set_halley_stop": (_c_int, [_vp, _c_int]),

@@ -37,14 +37,15 @@ def _key(sim, U):
         ",".join(str(v) for v in sim.flux), ",".join(str(k) for k in sim.bc_kinds))
 
 
-def tunable(sim):
-    """Whether the context's stage kernel has variants: the tile variant
-    selects the LF flux-splitting kernel (WENO5_JS or MUSCL) with the
-    per-cell temperature-solve stop; the Godunov and Steger-Warming kernels
-    and the grid-wide-stop kernel have one tile shape each."""
+def tunable(sim, U=None, theta=None):
+    """Whether the stage kernel has variants: the tile variant selects the LF
+    flux-splitting kernel (WENO5_JS or MUSCL) with the per-cell
+    temperature-solve stop; the Godunov and Steger-Warming kernels and the
+    grid-wide-stop kernel have one tile shape each.  With U, for U's grid: a
+    small one runs the compact kernel, whose tile follows from the grid."""
     solver, split = sim.flux[0], sim.flux[1]
     return (solver == _lib.SOLVER_TYPES["flux_splitting"] and split == _lib.SPLIT_METHODS["LF"]
-            and sim.halley_stop == "per_cell")
+            and sim.halley_stop == "per_cell" and (U is None or not sim.compact(U, theta)))
 
 
 def _load_file():
@@ -69,9 +70,9 @@ def tune(sim, U, aux, steps=8, theta=None, force=False):
     The caller's U and aux are not modified."""
     import torch
     U, aux = sim._state(U, aux)
-    if not tunable(sim):
+    if not tunable(sim, U, theta):
         return {"variant": sim.get_tile(U, theta), "tuned": False,
-                "reason": "this flux path / temperature-solve stop has one tile shape"}
+                "reason": "this grid, flux path or temperature-solve stop has one tile shape"}
     key = _key(sim, U)
     table = dict(_load_file())
     table.update(_MEM)

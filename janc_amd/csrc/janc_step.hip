@@ -1388,6 +1388,12 @@ int jh_tile_info(int variant, int* rows, int* threads, int* waves) {
   return JH_OK;
 }
 
+int jh_ctx_compact(const jh_ctx* c) {
+  return c && c->compact.R > 0 && c->solver == JH_SOLVER_FLUX_SPLITTING &&
+         c->split == JH_SPLIT_LF && c->recon == JH_RECON_WENO5_JS &&
+         c->halley == JH_HALLEY_PER_CELL;
+}
+
 int jh_ctx_get_tile(const jh_ctx* c) { return c ? c->tile : -1; }
 
 int jh_ctx_set_stream(jh_ctx* c, void* stream) {

@@ -504,6 +504,12 @@ class Simulator:
         ctx = self._context(U, theta)
         return int(ctx.lib.jh_ctx_get_tile(ctx.h))
 
+    def compact(self, U, theta=None):
+        """Whether the RK stages of U's grid run the compact kernel of small
+        grids (jh_ctx_compact) rather than a tile variant."""
+        ctx = self._context(U, theta)
+        return bool(ctx.lib.jh_ctx_compact(ctx.h))
+
     def autotune(self, U, aux, steps=8, theta=None, force=False):
         """Time every stage-kernel variant on a copy of (U, aux); keep the fastest."""
         from .autotune import tune

@@ -1,0 +1,43 @@
+"""Which stage kernel a context runs: the compact one on small grids."""
+import pytest
+
+from janc_amd import cases
+from janc_amd.autotune import variants
+from janc_amd.mechanism import Mechanism
+from janc_amd.solver import Simulator
+
+torch = pytest.importorskip("torch")
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+
+SIDES = ("left_boundary", "right_boundary", "bottom_boundary", "top_boundary")
+CHANNEL = dict(zip(SIDES, ("periodic", "periodic", "no_slip_wall", "slip_wall")))
+
+
+def _case(kind, nx, ny):
+    mech = Mechanism()
+    if kind == "annulus":
+        return cases.rdc_annulus(mech, nx=nx, ny=ny, seed_cols=nx // 5)
+    U, aux, g = cases.detonation_tube(mech, nx=nx, ny=ny, driver=nx // 8)
+    return U, aux, dict(g, boundary_config=CHANNEL), None
+
+
+@pytest.mark.parametrize("nx,ny,small", [(131, 77, True), (459, 467, False)])
+def test_autotune_times_variants_where_they_run(nx, ny, small, tmp_path, monkeypatch):
+    """A small grid has no variants to time: nothing is stored, in memory or in
+    the cache file, and the compact kernel stays."""
+    import janc_amd.autotune as at
+    path = tmp_path / "tune.json"
+    monkeypatch.setenv("JANC_AMD_TUNE_CACHE", str(path))
+    monkeypatch.setattr(at, "_MEM", {})
+    U, aux, g, _ = _case("channel", nx, ny)
+    U, aux = torch.as_tensor(U).cuda(), torch.as_tensor(aux).cuda()
+    sim = Simulator(cases.simulation_config(g, cfl=0.3))
+    t = sim.autotune(U, aux, steps=1)
+    assert at.tunable(sim) and at.tunable(sim, U) != small
+    assert sim.compact(U) == small
+    assert path.exists() != small and bool(at._MEM) != small
+    if small:
+        assert t["tuned"] is False and t["variant"] == sim.get_tile(U)
+    else:
+        assert sorted(int(k) for k in t["ms_per_step"]) == [v["variant"] for v in variants()]
