@@ -458,12 +458,14 @@ def _batch_leg(mech, steps, tune, torch):
     torch.cuda.synchronize()
     t_batch = time.perf_counter() - t0
     flags = b.health()
-    # sequential: one Simulator per case, same tile variant, warm contexts
+    # sequential: one Simulator per case with its own default kernel (the
+    # batch's tile variant where that is the wide one), warm contexts
     sims = [Simulator(c) for c in cfgs]
     Uq = [U.clone() for U in U0]
     Aq = [a.clone() for a in A0]
     for sim, U, a in zip(sims, Uq, Aq):
-        sim.set_tile(U, b.get_tile())
+        if not sim.compact(U):
+            sim.set_tile(U, b.get_tile())
         Uw, aw = U.clone(), a.clone()
         sim.advance(Uw, aw, 1)
     torch.cuda.synchronize()

@@ -110,8 +110,9 @@ int jh_ctx_set_flux(jh_ctx* ctx, int solver_type, int split_method, int reconstr
  * tile autotuner (janc_amd/autotune.py).  The Godunov kernel has one tile
  * shape per reconstruction (WENO5_JS: 64 x 3 cells, 256 threads; MUSCL:
  * 64 x 7 cells, 512 threads), the Steger-Warming kernel one (64 x 16 cells,
- * 512 threads).  Grids of up to 200000 cells run a kernel of smaller tiles
- * under LF splitting with WENO5_JS, whatever the variant.
+ * 512 threads).  Grids of up to 200000 cells run a kernel of smaller tiles by
+ * default under LF splitting with WENO5_JS, with the same results bit for bit;
+ * a context whose variant has been set runs that variant on any grid.
  * jh_ctx_compact: 1 if the context's RK stages run the kernel of smaller
  * tiles, 0 if not. */
 int jh_ctx_set_tile(jh_ctx* ctx, int variant);

@@ -243,8 +243,8 @@ int default_tile(int precision, long long tiles16, int recon = JH_RECON_WENO5_JS
 // rows at a 4-wave register budget, whatever the context's variant.
 constexpr int kGridRows = 16;
 
-// Small grids: the compact stage kernel (compact.hpp) by cell count, whatever
-// the tile variant (which shapes the wide kernel).  Up to 256 tiles of a wave
+// Small grids: the compact stage kernel (compact.hpp) by cell count, unless the
+// caller has chosen a variant of the wide kernel (jh_ctx_set_tile).  Up to 256 tiles of a wave
 // per variable all 12 variables run at once (14336 cells = one block per CU);
 // then two groups of rounds while the chip still holds every block at once
 // (50000 cells); then 2 groups of 256 threads, until the wide kernel has tiles
@@ -301,7 +301,7 @@ void launch_split_stage(jh_ctx* c, const StepArgs<Real>& a, int stage, const Rea
     return;
   }
   if constexpr (MODE == MODE_RK && RECON == RECON_WENO5) {
-    if (c->compact.R > 0) {
+    if (c->compact.R > 0 && !c->tile_chosen) {
       launch_compact<Real>(c, a, stage, Us, As, Un, Uo, Ao);
       return;
     }
@@ -1389,7 +1389,7 @@ int jh_tile_info(int variant, int* rows, int* threads, int* waves) {
 }
 
 int jh_ctx_compact(const jh_ctx* c) {
-  return c && c->compact.R > 0 && c->solver == JH_SOLVER_FLUX_SPLITTING &&
+  return c && c->compact.R > 0 && !c->tile_chosen && c->solver == JH_SOLVER_FLUX_SPLITTING &&
          c->split == JH_SPLIT_LF && c->recon == JH_RECON_WENO5_JS &&
          c->halley == JH_HALLEY_PER_CELL;
 }

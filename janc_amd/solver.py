@@ -496,7 +496,8 @@ class Simulator:
         return (gU, ga, Uo, ao) if with_output else (gU, ga)
 
     def set_tile(self, U, variant, theta=None):
-        """Select the stage-kernel variant (jh_ctx_set_tile) for U's grid."""
+        """Select the stage-kernel variant (jh_ctx_set_tile) for U's grid; a
+        small grid then runs it in place of the compact kernel."""
         ctx = self._context(U, theta)
         _lib.check(ctx.lib.jh_ctx_set_tile(ctx.h, int(variant)), ctx.h)
 

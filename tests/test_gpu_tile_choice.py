@@ -1,4 +1,8 @@
-"""Which stage kernel a context runs: the compact one on small grids."""
+"""Which stage kernel a context runs: the compact one on small grids by
+default, the chosen variant of the wide one after set_tile.  Every variant
+gives the default kernel's states and time steps bit for bit, on a small grid
+and on one past the compact kernel's range, with strips (inlet, outlet) and
+with source-cell halos (wall kinds, periodic)."""
 import pytest
 
 from janc_amd import cases
@@ -20,6 +24,29 @@ def _case(kind, nx, ny):
         return cases.rdc_annulus(mech, nx=nx, ny=ny, seed_cols=nx // 5)
     U, aux, g = cases.detonation_tube(mech, nx=nx, ny=ny, driver=nx // 8)
     return U, aux, dict(g, boundary_config=CHANNEL), None
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind,nx,ny,small", [("annulus", 131, 77, True), ("channel", 131, 77, True),
+                                              ("annulus", 459, 467, False),
+                                              ("channel", 459, 467, False)])
+def test_set_tile_runs_the_variant(kind, nx, ny, small, precision):
+    U0, aux0, g, theta = _case(kind, nx, ny)
+    dt = torch.float64 if precision == "fp64" else torch.float32
+    U0, aux0 = (torch.as_tensor(v).to(dtype=dt).cuda() for v in (U0, aux0))
+    sim = Simulator(cases.simulation_config(g, cfl=0.3, precision=precision, theta=theta))
+    assert sim.compact(U0, theta) == small
+    ref = [U0.clone(), aux0.clone()]
+    ref.append(sim.advance(ref[0], ref[1], 3, theta)[2])
+    for v in variants():
+        sim.set_tile(U0, v["variant"], theta)
+        assert not sim.compact(U0, theta) and sim.get_tile(U0, theta) == v["variant"]
+        U, aux = U0.clone(), aux0.clone()
+        hist = sim.advance(U, aux, 3, theta)[2]
+        torch.cuda.synchronize()
+        print(kind, nx, ny, precision, "variant", v, flush=True)
+        assert torch.isfinite(U).all()
+        assert torch.equal(U, ref[0]) and torch.equal(aux, ref[1]) and torch.equal(hist, ref[2])
 
 
 @pytest.mark.parametrize("nx,ny,small", [(131, 77, True), (459, 467, False)])
