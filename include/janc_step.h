@@ -110,11 +110,12 @@ int jh_ctx_set_flux(jh_ctx* ctx, int solver_type, int split_method, int reconstr
  * tile autotuner (janc_amd/autotune.py).  The Godunov kernel has one tile
  * shape per reconstruction (WENO5_JS: 64 x 3 cells, 256 threads; MUSCL:
  * 64 x 7 cells, 512 threads), the Steger-Warming kernel one (64 x 16 cells,
- * 512 threads).  Grids of up to 200000 cells run a kernel of smaller tiles by
- * default under LF splitting with WENO5_JS, with the same results bit for bit;
- * a context whose variant has been set runs that variant on any grid.
- * jh_ctx_compact: 1 if the context's RK stages run the kernel of smaller
- * tiles, 0 if not. */
+ * 512 threads).  Small grids (up to about 180000 cells) run a kernel of smaller
+ * tiles by default under LF splitting with WENO5_JS, with the same results bit
+ * for bit; a context whose variant has been set runs that variant on any grid.
+ * jh_ctx_compact: the number of thread groups (12, 6 or 2) that share out the
+ * variables if the context's RK stages run the kernel of smaller tiles, 0 if
+ * they do not. */
 int jh_ctx_set_tile(jh_ctx* ctx, int variant);
 int jh_ctx_get_tile(const jh_ctx* ctx);
 int jh_ctx_compact(const jh_ctx* ctx);

@@ -38,7 +38,8 @@ struct jh_ctx {
   bool user_filled[4] = {false, false, false, false};   // JH_BC_USER strips written
   int tile = 0;                   // stage-kernel variant (kTileRows / kTileWaves)
   bool tile_chosen = false;       // by jh_ctx_set_tile
-  CompactTile compact{0, 0, 0, 0};   // small grids: the compact kernel's tile (R = 0: none)
+  int rule = -1;                  // kCompactRules entry of a small grid, -1: wide kernel
+  CompactTile compact{0, 0, 0, 0};   // and its tile
   int solver = JH_SOLVER_FLUX_SPLITTING;   // jh_ctx_set_flux
   int split = JH_SPLIT_LF;
   int recon = JH_RECON_WENO5_JS;
@@ -243,24 +244,30 @@ int default_tile(int precision, long long tiles16, int recon = JH_RECON_WENO5_JS
 // rows at a 4-wave register budget, whatever the context's variant.
 constexpr int kGridRows = 16;
 
-// Small grids: the compact stage kernel (compact.hpp) by cell count, unless the
-// caller has chosen a variant of the wide kernel (jh_ctx_set_tile).  Up to 256 tiles of a wave
-// per variable all 12 variables run at once (14336 cells = one block per CU);
-// then two groups of rounds while the chip still holds every block at once
-// (50000 cells); then 2 groups of 256 threads, until the wide kernel has tiles
-// enough for the chip.  Microseconds per FP64 step (wide / compact, G = 12, 6,
-// 2): 4096 cells 155 / 46, 53, 66; 16384: 157 / 60, 58, 70; 25641: 160 / 62,
-// 61, 72; 65536: 166 / 109, 126, 97; 105000: 175 / 158, 165, 103; 262144: 191 /
-// 315, 349, 205.  Mixed: 4096: 121 / 45, 51, 65; 25641: 126 / 60, 59, 71; 65536:
-// 131 / 104, 118, 87; 105000: 139 / 142, 151, 93; 262144: 157 / 293, 322, 164.
-struct CompactRule { int groups, threads, halo; long long cells; };
-constexpr CompactRule kCompactRules[3] = {{12, 64, 2, 14336}, {6, 128, 2, 50000},
-                                          {2, 256, 1, 200000}};
+// Small grids: the compact stage kernel (compact.hpp), unless the caller has
+// chosen a variant of the wide kernel (jh_ctx_set_tile): the first rule whose
+// tiles of the grid are no more than its limit.  12 groups (a wave per
+// variable, one round of variables) and 6 groups while every CU has one block
+// at most; the 6-group kernel holds one a CU (143 registers, 12 waves), so past
+// that it goes round twice, and the 12-group kernel's second blocks share their
+// CU's issue.  2 groups up to three blocks a CU: a fourth and the wide kernel,
+// by then with tiles enough, is faster.  Microseconds per FP64 step with 12, 6
+// and 2 groups: 14336 cells (256, 128, 64 tiles) 47.5, 50.7, 62.1; 14400 (270,
+// 132, 64) 54.5, 51.0, 62.3; 28000 as 200 x 140 (6: 250 tiles) 55 and 66, as 280 x
+// 100 (260) 80 and 66; 50000 (450) 89 and 70.  With 2 groups and the wide
+// kernel: 57500 cells (250 tiles) 73, 132; 65536 (288) 88, 132; 130000 (558) 128,
+// 138; 180000 (765) 137, 149; 185000 (792) 160, 149; 200000 (850) 163, 153.
+// Mixed: 14336 47.4, 49.6, 60.2; 14400 53.2, 50.2, 61.2; 200 x 140 54 and 64, 280 x 100
+// 78 and 64; 2 groups and wide at 130000 118, 127, 180000 127, 139, 185000 141, 136.
+struct CompactRule { int groups, threads, halo, tiles; };
+constexpr CompactRule kCompactRules[3] = {{12, 64, 2, 256}, {6, 128, 2, 256}, {2, 256, 1, 768}};
 
-int compact_rule(const jh_ctx* c) {
-  const long long n = (long long)c->nx * c->ny;
-  for (int k = 0; k < 3; ++k)
-    if (n <= kCompactRules[k].cells) return k;
+// The rule of an nx x ny grid and its tile in ct; -1: the wide kernel.
+int compact_rule(int nx, int ny, CompactTile& ct) {
+  for (int k = 0; k < 3; ++k) {
+    ct = compact_tile(nx, ny, kCompactRules[k].threads, kCompactRules[k].halo);
+    if ((long long)ct.tiles_x * ct.tiles_y <= kCompactRules[k].tiles) return k;
+  }
   return -1;
 }
 
@@ -283,7 +290,7 @@ void launch_compact_rule(jh_ctx* c, const StepArgs<Real>& a, int stage, const Re
 template <typename Real>
 void launch_compact(jh_ctx* c, const StepArgs<Real>& a, int stage, const Real* Us, const Real* As,
                     const Real* Un, Real* Uo, Real* Ao) {
-  switch (compact_rule(c)) {
+  switch (c->rule) {
     case 0: launch_compact_rule<Real, 0>(c, a, stage, Us, As, Un, Uo, Ao); break;
     case 1: launch_compact_rule<Real, 1>(c, a, stage, Us, As, Un, Uo, Ao); break;
     case 2: launch_compact_rule<Real, 2>(c, a, stage, Us, As, Un, Uo, Ao); break;
@@ -301,7 +308,7 @@ void launch_split_stage(jh_ctx* c, const StepArgs<Real>& a, int stage, const Rea
     return;
   }
   if constexpr (MODE == MODE_RK && RECON == RECON_WENO5) {
-    if (c->compact.R > 0 && !c->tile_chosen) {
+    if (c->rule >= 0 && !c->tile_chosen) {
       launch_compact<Real>(c, a, stage, Us, As, Un, Uo, Ao);
       return;
     }
@@ -1235,9 +1242,7 @@ int jh_ctx_create(int nx, int ny, double dx, double dy, const int* bc_kind,
   c->dy = dy;
   c->precision = precision;
   c->tile = ctx_default_tile(c);
-  const int rule = compact_rule(c);
-  if (rule >= 0)
-    c->compact = compact_tile(nx, ny, kCompactRules[rule].threads, kCompactRules[rule].halo);
+  c->rule = compact_rule(nx, ny, c->compact);
   c->stream = static_cast<hipStream_t>(stream);
   for (int s = 0; s < 4; ++s) {
     c->bc[s] = bc_kind[s];
@@ -1389,9 +1394,10 @@ int jh_tile_info(int variant, int* rows, int* threads, int* waves) {
 }
 
 int jh_ctx_compact(const jh_ctx* c) {
-  return c && c->compact.R > 0 && !c->tile_chosen && c->solver == JH_SOLVER_FLUX_SPLITTING &&
-         c->split == JH_SPLIT_LF && c->recon == JH_RECON_WENO5_JS &&
-         c->halley == JH_HALLEY_PER_CELL;
+  const bool on = c && c->rule >= 0 && !c->tile_chosen &&
+                  c->solver == JH_SOLVER_FLUX_SPLITTING && c->split == JH_SPLIT_LF &&
+                  c->recon == JH_RECON_WENO5_JS && c->halley == JH_HALLEY_PER_CELL;
+  return on ? kCompactRules[c->rule].groups : 0;
 }
 
 int jh_ctx_get_tile(const jh_ctx* c) { return c ? c->tile : -1; }

@@ -68,3 +68,26 @@ def test_autotune_times_variants_where_they_run(nx, ny, small, tmp_path, monkeyp
         assert t["tuned"] is False and t["variant"] == sim.get_tile(U)
     else:
         assert sorted(int(k) for k in t["ms_per_step"]) == [v["variant"] for v in variants()]
+
+
+@pytest.mark.parametrize("nx,ny,groups", [(4, 4, 12), (128, 112, 12), (120, 120, 6), (200, 140, 6),
+                                          (2000, 14, 6), (280, 100, 2), (200, 150, 2),
+                                          (250, 200, 2), (3000, 60, 2), (720, 250, 2),
+                                          (740, 250, 0), (400, 500, 0)])
+def test_compact_rule_goes_by_tiles(nx, ny, groups):
+    """12 and 6 groups only while their tiles are at most one for each of the
+    256 CUs, 2 groups up to three; each form equals the wide kernel."""
+    mech = Mechanism()
+    U0, aux0, g = cases.detonation_tube(mech, nx=nx, ny=ny, driver=max(1, nx // 8))
+    for precision, dt in (("fp64", torch.float64), ("mixed", torch.float32)):
+        Ui, ai = (torch.as_tensor(v).to(dtype=dt).cuda() for v in (U0, aux0))
+        sim = Simulator(cases.simulation_config(g, cfl=0.3, precision=precision))
+        ctx = sim._context(Ui, None)
+        assert ctx.lib.jh_ctx_compact(ctx.h) == groups
+        out = []
+        for _ in range(2):
+            U, aux = Ui.clone(), ai.clone()
+            out.append((U, aux, sim.advance(U, aux, 2)[2]))
+            sim.set_tile(Ui, sim.get_tile(Ui))
+        assert torch.isfinite(out[0][0]).all()
+        assert all(torch.equal(a, b) for a, b in zip(*out))
