@@ -24,7 +24,9 @@ namespace jh {
 // place) takes 694 us at 256 or 384 threads, 745 at 512, 799 at 192; the mixed
 // step of 1000 blocks of 40 x 50 943 us at 256, 954 at 192, 1145 at 512.
 constexpr int kBlkThreads = 256;
-// Waves per SIMD its register budget allows (FP32 needs 80 registers).
+// Waves per SIMD its register budget allows.  FP32 takes 85 registers; held to 80 for
+// the sixth wave it spills 3 of them (16 bytes a lane) and is the faster: the mixed
+// level above 960 us with four or five, 939 with six.
 template <typename Real> struct BlkWaves { static constexpr int value = 4; };
 template <> struct BlkWaves<float> { static constexpr int value = 6; };
 

@@ -13,9 +13,9 @@
 // fluxes, a face's WENO, the temperature solve), so the chain is made as short
 // as the variables allow; on AMR levels FP64 / FP32 issue, so the tile is made
 // to fill its waves (one cell, one x face and one y face per thread).  Whole
-// steps, before and after: 128 x 32 FP64 155 -> 46 us, 256 x 64 mixed 122 -> 54
-// us; a level of 2500 FP64 blocks of 20 x 20 2276 -> 705 us, of 1000 mixed
-// blocks of 40 x 50 1608 -> 946 us.
+// steps, before and after: 128 x 32 FP64 155 -> 46 us, 256 x 64 mixed 122 -> 49
+// us; a level of 2500 FP64 blocks of 20 x 20 2276 -> 659 us, of 1000 mixed
+// blocks of 40 x 50 1608 -> 938 us.
 #pragma once
 #include <hip/hip_runtime.h>
 

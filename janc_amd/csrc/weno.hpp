@@ -84,8 +84,9 @@ __host__ __device__ __forceinline__ double weno5_lf(double p0, double p1, double
 // kPairMax the quotients are taken one by one (finite up to jumps of 6e33).  Below
 // it nothing overflows: |nL| <= 4 d dL with d the largest difference, and dL dR >=
 // 1e-37 d^4, so d < 1e60.  The branch also keeps the compiler from working on several
-// variables at once: 154 -> 118 registers, four waves per SIMD instead of three (HLLC step of
-// 1500 x 300 cells: 401 -> 378 us; the stage 119 us with two reciprocals, 111 with one).
+// variables at once: 154 -> 118 registers, four waves per SIMD instead of three (HLLC
+// stage of 1500 x 300 cells: 119 us with two reciprocals, 111 with one, 105 with the
+// branch; the step 399 -> 377).
 constexpr double kPairMax = 1e200;
 __host__ __device__ __forceinline__ void weno5_LR(double v0, double v1, double v2, double v3,
                                                   double v4, double v5, double& L, double& R) {
@@ -192,7 +193,8 @@ namespace jh {
 // (the reverse mode of WENO5_JS.py:17-33 as JAX differentiates it):
 //   dq/dv_j = sum_k w_k dq_k/dv_j + sum_k kappa_k de_k/dv_j,
 //   kappa_k = -2 w_k (q_k - q) / e_k,  e_k = eps + IS_k,
-// in weno5's difference form (q_k - q = c_k - sum_m w_m c_m), with the three
+// in the first and second differences of the FP32 weno5 above (q_k - q = c_k - sum_m
+// w_m c_m; the FP64 value itself is taken from completed squares), with the three
 // 1/e_k from 1/(e_1 e_2 e_3) and the weights' normaliser from the same
 // reciprocal (e^7 stays in FP64 range for any e = eps + IS_k the split
 // fluxes produce: 1e-42 at eps, 1e154 at IS = 1e22).  With A_k the halved first-
