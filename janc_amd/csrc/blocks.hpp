@@ -71,8 +71,8 @@ __global__ __launch_bounds__(256) void blocks_alpha_kernel(StepArgs<Real> a, int
 // interior: the compact stage body on a block's padded planes, the block's
 // own maxima.  Jobs (block, tile) in XCD-contiguous order.  bs / bo: block
 // strides of the inputs and of the output (12 planes per block for MODE_RHS).
-// Bound by FP64 issue; the 64-column tile it replaced left 44 of 64 lanes of a
-// 20 x 20 block idle.
+// Bound by FP64 issue; the 64-column tile of the wide body leaves 44 of 64 lanes of
+// a 20 x 20 block idle.
 template <typename Real, int MODE>
 __global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(BlkWaves<Real>::value)))
 void blocks_stage_kernel(StepArgs<Real> a, CompactTile ct, int stage, long long bs, long long bo,
@@ -91,6 +91,28 @@ void blocks_stage_kernel(StepArgs<Real> a, CompactTile ct, int stage, long long 
   compact_body<Real, MODE, 1, 1, ADDR_PAD>(ab, ct, stage, Us, Us + NU * P, Bn + (size_t)b * bs, Uo,
                                            Uo + NU * P, tile, blockDim.x,
                                            reinterpret_cast<Real*>(dyn), mix, red);
+}
+
+// The same by the wide stage body on kBlkRows x 64 tiles, bit for bit: for many blocks
+// that fill its columns (blocks_wide).  Fewer halo cells a cell, and in FP32 runs of
+// faces that share their differences: a mixed stage of 256 blocks of 64 x 64 takes 137
+// us with it and 159 with compact tiles, an FP64 one 188 and 211.
+constexpr int kBlkRows = 8;
+template <typename Real, int MODE>
+__global__ __launch_bounds__(Tile<kBlkRows>::NT) __attribute__((amdgpu_waves_per_eu(4)))
+void blocks_stage_wide_kernel(StepArgs<Real> a, int stage, int tiles, long long bs, long long bo,
+                              const Real* Bs, const Real* Bn, Real* Bo) {
+  __shared__ StageLds<Real, kBlkRows> L;
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  const int b = t / tiles, tile = t - b * tiles;
+  const size_t P = (size_t)(a.nx + 6) * (a.ny + 6);
+  StepArgs<Real> ab = a;
+  ab.sc = a.sc + b;
+  ab.parity = 0;
+  const Real* Us = Bs + (size_t)b * bs;
+  Real* Uo = Bo + (size_t)b * bo;
+  stage_body<Real, MODE, kBlkRows, RECON_WENO5, SPLIT_LF, Real, false, false, true>(
+      ab, stage, Us, Us + NU * P, Bn + (size_t)b * bs, Uo, Uo + NU * P, tile, L);
 }
 
 // One RK stage of a uniform level's blocks read in place: the halo of a block

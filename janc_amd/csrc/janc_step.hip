@@ -1029,6 +1029,7 @@ void drop_graph(jh_batch* b) {
 
 struct jh_blocks {
   int nx = 0, ny = 0;                 // block interior
+  CompactTile ct{0, 0, 0, 0};         // and its compact tile
   double dx = 0, dy = 0;
   int precision = JH_PREC_FP64;
   hipStream_t stream = nullptr;
@@ -1118,6 +1119,22 @@ int blk_threads(const CompactTile& ct) {
   return (m + 63) / 64 * 64;
 }
 
+int wide_tiles(const jh_blocks* b) {
+  return ((b->nx + kBlkRows - 1) / kBlkRows) * ((b->ny + TY - 1) / TY);
+}
+// Whether padded blocks take the wide stage body: where their rows fill 64 columns, so
+// that compact tiles are more than twice as many, and the wide tiles are at least two a
+// CU.  A stage with the compact over one with the wide body, FP64 and mixed, a million
+// cells: 64 x 64 (20 tiles for 8) 1.06 and 1.11, 64 x 128 (36 for 16) 1.02 and 1.08, 32 x
+// 500 (68 for 32) 1.03 and 1.04; two for one and less: 32 x 120 (16 for 8) 0.98 and 0.99,
+// 64 x 104 (28 for 16) 0.89 and 0.94, 20 x 40 (4 for 3) 0.82 and 0.79.  Blocks of 64 x 64: 8 of
+// them (64 wide tiles) 0.76 and 0.82, 32 (256) 0.98 and 0.98, 64 (512) 1.04 and 1.04, 512
+// 1.16 and 1.19.
+bool blocks_wide(const jh_blocks* b, int n_blk) {
+  const int wide = wide_tiles(b);
+  return b->ct.tiles_x * b->ct.tiles_y > 2 * wide && (long long)n_blk * wide >= 512;
+}
+
 template <typename Real, int MODE>
 int blocks_stage_impl(jh_blocks* b, int n_blk, int stage, const Real* Bs, const Real* Bn,
                       Real* Bo, double dt, StepScalars* sc) {
@@ -1126,10 +1143,16 @@ int blocks_stage_impl(jh_blocks* b, int n_blk, int stage, const Real* Bs, const 
   auto a = blocks_args<Real>(b, dt, sc);
   hipStream_t st = b->stream;
   blocks_alpha_kernel<Real><<<n_blk, 256, 0, st>>>(a, stage, bs, Bs);
-  const CompactTile ct = compact_tile(b->nx, b->ny, kBlkThreads, 1);
-  blocks_stage_kernel<Real, MODE>
-      <<<n_blk * ct.tiles_x * ct.tiles_y, blk_threads(ct), compact_lds<1>(ct) * sizeof(Real), st>>>(
-          a, ct, stage, bs, bo, Bs, Bn, Bo);
+  if (blocks_wide(b, n_blk)) {
+    const int tiles = wide_tiles(b);
+    blocks_stage_wide_kernel<Real, MODE>
+        <<<n_blk * tiles, Tile<kBlkRows>::NT, 0, st>>>(a, stage, tiles, bs, bo, Bs, Bn, Bo);
+  } else {
+    const CompactTile& ct = b->ct;
+    blocks_stage_kernel<Real, MODE>
+        <<<n_blk * ct.tiles_x * ct.tiles_y, blk_threads(ct), compact_lds<1>(ct) * sizeof(Real),
+           st>>>(a, ct, stage, bs, bo, Bs, Bn, Bo);
+  }
   const int nring = (int)(P - (long long)b->nx * b->ny);
   blocks_ring_kernel<Real, MODE>
       <<<dim3((nring + 255) / 256, n_blk), 256, 0, st>>>(a, stage, bs, bo, Bs, Bn, Bo);
@@ -1167,7 +1190,7 @@ int level_step_impl(jh_blocks* b, int n_blk, const Real* blk, long long sb, long
                     reinterpret_cast<double*>(work + 2 * ss + sp)};
   hipStream_t st = b->stream;
   const auto a = blocks_args<Real>(b, dt, b->sc);
-  const CompactTile ct = compact_tile(b->nx, b->ny, kBlkThreads, 1);
+  const CompactTile& ct = b->ct;
   const int nb = n_blk * ct.tiles_x * ct.tiles_y, nt = blk_threads(ct);
   const size_t lds = compact_lds<1>(ct) * sizeof(Real);
   level_speeds_kernel<Real><<<n_blk, 256, 0, st>>>(a, sb, sv, sr, blk, spd[0], ncell);
@@ -1933,6 +1956,7 @@ int jh_blocks_create(int bnx, int bny, double dx, double dy, int precision, cons
   jh_blocks* b = new jh_blocks();
   b->nx = bnx;
   b->ny = bny;
+  b->ct = compact_tile(bnx, bny, kBlkThreads, 1);
   b->dx = dx;
   b->dy = dy;
   b->precision = precision;

@@ -1070,9 +1070,11 @@ struct StageLds {
 // RK combine (Real, the storage type, unless stated); GRID the grid-wide
 // temperature-solve stop (StepArgs::hside set), compiled separately so the
 // per-cell kernels keep their register budget; MIRROR the halo is read from the
-// source cells of copy-kind sides (locate_src).
+// source cells of copy-kind sides (locate_src); PAD the state planes are one
+// AMR block with its own ghost layers ((nx + 6) x (ny + 6), no ghost strips, no
+// next-stage maxima: the next stage's ghosts come from the caller).
 template <typename Real, int MODE, int TX, int RECON = RECON_WENO5, int SPLIT = SPLIT_LF,
-          typename W = Real, bool GRID = false, bool MIRROR = false>
+          typename W = Real, bool GRID = false, bool MIRROR = false, bool PAD = false>
 __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
                                            const Real* __restrict__ Us,
                                            const Real* __restrict__ auxs, const Real* Un,
@@ -1096,7 +1098,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
 
   const MechConst& c = *a.mc;
   if (MODE != MODE_RHS) load_mix_tables(c, L.mix);   // read after the phase barriers
-  const int nx = a.nx, ny = a.ny, n = nx * ny;
+  const int nx = a.nx, ny = a.ny, n = PAD ? (nx + 6) * (ny + 6) : nx * ny;
   // the wave index through readfirstlane: the tile rows, slots and face
   // runs derived from it are wave-uniform to the compiler (scalar registers
   // and branches)
@@ -1173,7 +1175,8 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
 #pragma unroll
   for (int s = 0; s < NSL; ++s) {
     unsigned int f = 0u;
-    if constexpr (MIRROR) ref[s] = locate_src<Real>(a, Us, auxs, gxs[s], gys[s], f);
+    if constexpr (PAD) ref[s] = locate_padded<Real>(a, Us, auxs, gxs[s], gys[s]);
+    else if constexpr (MIRROR) ref[s] = locate_src<Real>(a, Us, auxs, gxs[s], gys[s], f);
     else ref[s] = locate<Real>(a, Us, auxs, gxs[s], gys[s]);
     if (!has[s]) ref[s].ok = false;
     if constexpr (kOff) off[s] = (unsigned int)((ref[s].u - Us) * sizeof(Real));
@@ -1199,7 +1202,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     own[s] = gxs[s] < nx && gys[s] < ny;
-    oidx[s] = gxs[s] * ny + gys[s];
+    oidx[s] = PAD ? (gxs[s] + 3) * (ny + 6) + gys[s] + 3 : gxs[s] * ny + gys[s];
   }
   const auto own_at = [&](auto* base, int v, int s) -> auto& {   // own cell s of plane v
     if constexpr (kScalar)
@@ -1399,7 +1402,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
     own_at(auxo, 0, s) = (Real)gamma;
     own_at(auxo, 1, s) = (Real)T;
     fl |= halley_flags(rho, e, R, T, gamma, conv);
-    if (stage < 2) {
+    if (!PAD && stage < 2) {
       // next stage's alpha from the stored (rounded) values
       const double gs = (double)(Real)gamma, Ts = (double)(Real)T;
       const double p = rho * R * Ts;
@@ -1423,7 +1426,7 @@ __device__ __forceinline__ void stage_body(const StepArgs<Real>& a, int stage,
     // (the reduction's first barrier)
     block_max_bits_multi<NT, kGridSlotsStage>(gv, &a.sc->gs[a.parity][stage].nstar,
                                               reinterpret_cast<unsigned long long*>(&L.Hxp[0][0]));
-  } else if (stage < 2) {
+  } else if (!PAD && stage < 2) {
     const unsigned long long m[2] = {dbits(mx), dbits(my)};
     block_max_to<NT, 2>(m, [&](int k) { return &a.sc->amax[a.parity][stage + 1][k]; }, L.red);
   }
